@@ -46,6 +46,7 @@ typedef struct ihipStream_t* sluice_stream_t; /* == hipStream_t */
 #define SLUICE_MAX_TOPK 16       /* k */
 #define SLUICE_MAX_PAIRS 4096    /* T*k (token, expert) pairs per call */
 #define SLUICE_BLOCK_M 16        /* tokens per aligned block */
+#define SLUICE_MAX_PREFILL_PAIRS 65536 /* pairs per sluice_fused_experts_prefill call */
 
 #define SLUICE_ABI_VERSION 1
 
@@ -196,6 +197,20 @@ int sluice_fused_experts_fp8(const void* x, const void* w13,
                              int shared_I, const void* shared, void* workspace,
                              size_t workspace_bytes, void* out, const int32_t* plan,
                              sluice_stream_t stream);
+
+/* The same product for prefill chunks of more than SLUICE_MAX_PAIRS pairs:
+ * T*(k + shared_I/I) <= SLUICE_MAX_PREFILL_PAIRS in one call, so that the
+ * chunk reads each expert's weights once.  bf16 experts when w13_scale and
+ * w2_scale are NULL, e4m3fn with 128x128 block scales when both are given.
+ * Workspace: sluice_fused_experts_workspace() bytes, as above. */
+int sluice_fused_experts_prefill(const void* x, const void* w13, const float* w13_scale,
+                                 const void* w2, const float* w2_scale, const float* topk_w,
+                                 const int32_t* topk_ids, const int32_t* expert_map, int T, int H,
+                                 int I, int k, int E, int S, float scale, const void* shared_w13,
+                                 const float* shared_w13_scale, const void* shared_w2,
+                                 const float* shared_w2_scale, int shared_I, const void* shared,
+                                 void* workspace, size_t workspace_bytes, void* out,
+                                 sluice_stream_t stream);
 
 /* Token permute / align-to-block (vLLM moe_align_block_size): groups the
  * T*k (token, expert) pairs by slot into blocks of <= SLUICE_BLOCK_M pairs,

@@ -33,6 +33,7 @@ MAX_EXPERTS = 1024
 MAX_SLOTS = 512
 MAX_TOPK = 16
 MAX_PAIRS = 4096
+MAX_PREFILL_PAIRS = 65536
 BLOCK_M = 16
 
 # Every symbol include/sluice.h declares: name -> (restype, argtypes).
@@ -64,6 +65,11 @@ SIGNATURES = {
         c_int,
         [_P, _P, _P, _P, _P, c_int, c_int, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int,
          c_float, _P, _P, _P, _P, c_int, _P, _P, c_size_t, _P, _P, _P],
+    ),
+    "sluice_fused_experts_prefill": (
+        c_int,
+        [_P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_float, _P, _P,
+         _P, _P, c_int, _P, _P, c_size_t, _P, _P],
     ),
     "sluice_moe_plan_ints": (c_size_t, [c_int, c_int]),
     "sluice_read_probe": (c_int, [_P, c_size_t, _P, _P]),

@@ -74,7 +74,8 @@ def _run(cmd: list[str]) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"command failed ({r.returncode}): {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
-    noise = ("is not a recognized feature for this target", RESOURCE_REMARKS)
+    noise = ("is not a recognized feature for this target", RESOURCE_REMARKS,
+             "In file included from")
     for line in (r.stdout + r.stderr).splitlines():
         if line.strip() and not any(n in line for n in noise) and not line.lstrip().startswith(
                 ("|", "^")) and not re.match(r"^\s*\d+ \|", line):
@@ -82,8 +83,9 @@ def _run(cmd: list[str]) -> str:
     return r.stdout + r.stderr
 
 
-# Room the split launch of the expert product must leave per SIMD.  Its
-# pending workgroups wait for slots while the copies that fill them run.  The
+# Room the split launch of the expert product (and the tiled product, whose
+# persistent workgroups fill the device) must leave per SIMD.  Their
+# workgroups wait for slots while the copies that fill them run.  The
 # gap's copies go to the SDMA engines, but a host-to-device copy that runs as
 # a kernel (a HIP-stream copy of small host rows, or any copy with SDMA
 # switched off in the runtime) is one 512-thread workgroup (two waves per
@@ -93,7 +95,7 @@ def _run(cmd: list[str]) -> str:
 # and the waits would run to their bound.
 VGPR_FILE = 512
 COPY_KERNEL_VGPRS_PER_SIMD = 2 * 16
-WAITING_KERNELS = ("moe_gemm2_split_kernel",)
+WAITING_KERNELS = ("moe_gemm2_split_kernel", "moe_tile_kernel")
 # The gap server's decode of a coded expert (csrc/codec_kernel.hip) runs while the
 # split launch's pending workgroups wait for it: one 256-thread workgroup
 # (one wave per SIMD) must fit beside their waves.  Coded stores hold bf16

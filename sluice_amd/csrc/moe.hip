@@ -17,7 +17,8 @@
 // Launch shape: align (1 WG) -> gemm1 (+silu*up) -> gemm2 (*w) -> combine,
 // grid-stride kernels over a plan in global memory; the align launch is
 // skipped when the caller hands in the plan its router-split gap kernel
-// built.  (A single persistent kernel with cross-workgroup hand-offs was
+// built.  Calls with many tokens per expert (prefill chunks) run the tiled
+// product of tile.h instead.  (A single persistent kernel with cross-workgroup hand-offs was
 // measured 1.6-1.8x slower than these launches and is not kept.)
 #include <math.h>
 
@@ -858,6 +859,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(
   combine4<SPEC>(partial, valid, t, T, k, n_sh, H, h, scale, shared, out);
 }
 
+#include "tile.h"
+
 // ---------------------------------------------------------------------------
 // Host side.
 // ---------------------------------------------------------------------------
@@ -947,13 +950,13 @@ int wait_grid(K kernel, WaitKernel kind, int* out) {
 // The align kernel stages the map of all E experts in LDS.
 int check_common(int T, int H, int I, int k, int E, int S, int n_sh, const void* x,
                  const void* w13, const void* w2, const float* tw, const int32_t* ti,
-                 const void* shared, void* ws, size_t ws_bytes, void* out) {
+                 const void* shared, void* ws, size_t ws_bytes, void* out,
+                 long max_pairs = SLUICE_MAX_PAIRS) {
   if (T < 0 || H <= 0 || I <= 0 || k <= 0 || k > SLUICE_MAX_TOPK || E <= 0 ||
       E > SLUICE_MAX_EXPERTS || S <= 0 || S > SLUICE_MAX_SLOTS)
     return SLUICE_E_INVAL;
-  if ((long)T * k > SLUICE_MAX_PAIRS) return SLUICE_E_INVAL;
-  if (n_sh < 0 || n_sh > kMaxShared || (long)T * (k + n_sh) > SLUICE_MAX_PAIRS)
-    return SLUICE_E_INVAL;
+  if ((long)T * k > max_pairs) return SLUICE_E_INVAL;
+  if (n_sh < 0 || n_sh > kMaxShared || (long)T * (k + n_sh) > max_pairs) return SLUICE_E_INVAL;
   if (H % 64 != 0 || I % 64 != 0) return SLUICE_E_INVAL;
   if (T == 0) return SLUICE_OK;
   if (!x || !w13 || !w2 || !tw || !ti || !ws || !out) return SLUICE_E_INVAL;
@@ -976,6 +979,112 @@ int launch_combine(const float* partial, const int32_t* valid, int T, int k, int
   return (int)hipGetLastError();
 }
 
+// Tile shapes: 128 weight rows x BM pairs, four waves of 32 rows each.  As
+// many stages as let two workgroups share a CU's LDS; two independent
+// workgroups hide each other's barriers (one 8-wave workgroup of 256 rows
+// measured the same or slower: 372-428 against 338-395 us for gemm1 at 4096
+// tokens of the Qwen3 shape).
+template <bool FP8, bool G1, int BM>
+struct TileFor {
+  using type = TileCfg<FP8, G1, 128, BM, 4, 1, BM == 128 ? 2 : FP8 ? (BM == 64 ? 2 : 3)
+                                                                   : (BM == 64 ? 3 : 4)>;
+};
+template <>
+struct TileFor<false, false, 128> {  // short K (I): 219 against 238 us
+  using type = TileCfg<false, false, 256, 128, 4, 2, 3>;
+};
+
+// Pairs per tile, or 0 for the decode kernels, from the mean pairs per slot.
+// The decode kernels read an expert's weights once per 16 of its tokens and
+// so win while most experts have one block; at 12 pairs per slot the tiles
+// took over (us, decode kernels / tiles: V2-Lite 48 slots 177 / 187 at 12
+// with even routing and 207 / 188 with Zipf, 204 / 186 at 16; Qwen3 256 /
+// 246 at 12; V3 fp8 610 / 586 at 8, 701 / 612 at 12).  Larger tiles reuse
+// the weights more and pad more: 32 / 64 / 128 pairs gave 186 / 195 / 234 at
+// 16 per slot, 255 / 215 / 246 at 64, 385 / 289 / 267 at 128 (V2-Lite).
+//
+// A call over few slots must also fill the device: the tiles are taken where
+// they make at least one item per CU.
+template <bool FP8>
+int tile_pairs(const CallShape& cs, int E, int S) {
+  const int slots = std::min(E, S), P = cs.T * cs.k;
+  if (P > SLUICE_MAX_PAIRS || P >= 12 * slots) {
+    const int bm = FP8 ? (P < 32 * slots ? 32 : 64) : P < 20 * slots ? 32 : P < 100 * slots ? 64 : 128;
+    const long items = (long)std::max(P / bm, slots) * std::min(cs.I / 64, cs.H / 128);
+    if (P > SLUICE_MAX_PAIRS || items >= 256) return bm;
+  }
+  return 0;
+}
+
+// Workgroups of a persistent tile launch: as many as fit the device at once
+// (a multiple of 8: the XCDs), looked up once per device and kernel.
+template <typename C>
+int tile_grid(long items, int* out) {
+  static std::atomic<int> cache[kWaitDevices];
+  int dev = 0;
+  SLUICE_HIP_CHECK(hipGetDevice(&dev));
+  if (dev < 0 || dev >= kWaitDevices) return SLUICE_E_INVAL;
+  int n = cache[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    int per_cu = 0, cus = 0;
+    SLUICE_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, moe_tile_kernel<C>,
+                                                                  64 * C::NW, 0));
+    SLUICE_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    n = std::max(std::max(per_cu, 1) * std::max(cus, 1) / 8 * 8, 8);
+    cache[dev].store(n, std::memory_order_relaxed);
+  }
+  *out = (int)std::min<long>(n, (items + 7) / 8 * 8);
+  return SLUICE_OK;
+}
+
+template <typename C>
+int launch_tiles(const TileArgs& a, long tiles, hipStream_t st) {
+  const int n_out = C::G1 ? a.cs.I : a.cs.H;
+  int grid = 0;
+  const int rc = tile_grid<C>(tiles * ((n_out + C::kOut - 1) / C::kOut), &grid);
+  if (rc != SLUICE_OK) return rc;
+  hipLaunchKernelGGL(moe_tile_kernel<C>, dim3(grid), dim3(64 * C::NW), 0, st, a);
+  return (int)hipGetLastError();
+}
+
+template <bool FP8, int BM>
+int run_tiles(const TileArgs& a, long tiles, hipStream_t st) {
+  const int rc = launch_tiles<typename TileFor<FP8, true, BM>::type>(a, tiles, st);
+  if (rc != SLUICE_OK) return rc;
+  return launch_tiles<typename TileFor<FP8, false, BM>::type>(a, tiles, st);
+}
+
+// The tiled product: sort, gemm1, gemm2, combine.  The sorted call sits in
+// the workspace's plan area, which is always larger: the records, order and
+// flags take at most 7 ints per pair (+ 2048 for the slots' partial tiles,
+// when P > SLUICE_MAX_PAIRS), the plan 19.
+template <bool FP8>
+int run_tiled(const void* x, const ExpertW& W, const float* tw, const int32_t* ti,
+              const int32_t* map, const CallShape& cs, int E, int S, int n_sh, int bm, float scale,
+              const void* shared, const Workspace& w, void* out, hipStream_t st) {
+  const int T = cs.T, P = T * cs.k, P2 = P + n_sh * T;
+  const long tiles = tile_bound(P, std::min(E, S), T, n_sh, bm);
+  TilePlan pl;
+  pl.hdr = w.plan;
+  pl.tiles = (TileRec*)(w.plan + kPlanHeader);
+  pl.order = (int32_t*)(pl.tiles + tiles);
+  pl.valid = pl.order + P2;
+  if ((size_t)(pl.valid + P - w.plan) > plan_ints(P)) return SLUICE_E_INVAL;
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kSortThreads), 0, st, ti, P, map, E, S,
+                     W.wait.pending, T, n_sh, bm, pl);
+  SLUICE_HIP_CHECK(hipGetLastError());
+  const TileArgs a{(const uint16_t*)x, W, pl, cs, tw, w.act, w.partial};
+  int rc = SLUICE_OK;
+  if (bm == 32)
+    rc = run_tiles<FP8, 32>(a, tiles, st);
+  else if (FP8 || bm == 64)
+    rc = run_tiles<FP8, 64>(a, tiles, st);
+  else
+    rc = run_tiles<FP8, FP8 ? 64 : 128>(a, tiles, st);
+  if (rc != SLUICE_OK) return rc;
+  return launch_combine(w.partial, pl.valid, T, cs.k, n_sh, cs.H, scale, shared, out, st);
+}
+
 // plan: a plan of these ids over this map built on the stream before the
 // call (by the layer's gap kernel), or nullptr: the align kernel builds one
 // in the workspace.
@@ -990,6 +1099,9 @@ int run_experts(const void* x, const ExpertW& W, const float* tw, const int32_t*
   const CallShape cs{T, k, H, I};
   ExpertW Ww = W;
   if (map != nullptr) Ww.wait = slotwait_lookup(map);
+  const int bm = plan == nullptr ? tile_pairs<FP8>(cs, E, S) : 0;
+  if (bm > 0)
+    return run_tiled<FP8>(x, Ww, tw, ti, map, cs, E, S, n_sh, bm, scale, shared, w, out, st);
   if (plan == nullptr) {
     hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(kThreads), 0, st, ti, P, map, E, S,
                        Ww.wait.pending, w.plan);
@@ -1165,6 +1277,31 @@ extern "C" int sluice_fused_experts_fp8(const void* x, const void* w13, const fl
                   shared_w2_scale, S, shared_I};
   return run_experts<true>(x, W, topk_w, topk_ids, expert_map, T, H, I, k, E, S, n_sh, scale,
                            shared, workspace, plan, out, (hipStream_t)stream);
+}
+
+extern "C" int sluice_fused_experts_prefill(
+    const void* x, const void* w13, const float* w13_scale, const void* w2, const float* w2_scale,
+    const float* topk_w, const int32_t* topk_ids, const int32_t* expert_map, int T, int H, int I,
+    int k, int E, int S, float scale, const void* shared_w13, const float* shared_w13_scale,
+    const void* shared_w2, const float* shared_w2_scale, int shared_I, const void* shared,
+    void* workspace, size_t workspace_bytes_, void* out, sluice_stream_t stream) {
+  const bool fp8 = w13_scale != nullptr;
+  if (fp8 != (w2_scale != nullptr)) return SLUICE_E_INVAL;
+  if (fp8 && (H % kFp8Blk != 0 || I % kFp8Blk != 0)) return SLUICE_E_INVAL;
+  int n_sh = 0;
+  int rc = shared_groups(shared_I, I, shared_w13, shared_w2, &n_sh);
+  if (rc != SLUICE_OK) return rc;
+  if (fp8 && n_sh > 0 && (shared_w13_scale == nullptr || shared_w2_scale == nullptr))
+    return SLUICE_E_INVAL;
+  rc = check_common(T, H, I, k, E, S, n_sh, x, w13, w2, topk_w, topk_ids, shared, workspace,
+                    workspace_bytes_, out, SLUICE_MAX_PREFILL_PAIRS);
+  if (rc != SLUICE_OK || T == 0) return rc;
+  const ExpertW W{(const uint8_t*)w13, (const uint8_t*)w2, w13_scale, w2_scale,
+                  (const uint8_t*)shared_w13, (const uint8_t*)shared_w2, shared_w13_scale,
+                  shared_w2_scale, S, shared_I};
+  auto run = fp8 ? run_experts<true> : run_experts<false>;
+  return run(x, W, topk_w, topk_ids, expert_map, T, H, I, k, E, S, n_sh, scale, shared, workspace,
+             nullptr, out, (hipStream_t)stream);
 }
 
 extern "C" int sluice_moe_gemm1_bf16(const void* x, const void* w13, const int32_t* plan, int T,

@@ -26,6 +26,8 @@ from sluice_amd import _lib
 
 _SCORING = {"softmax": 0, "sigmoid": 1}
 _MAX_PAIRS = 4096  # SLUICE_MAX_PAIRS: (token, expert) pairs per fused_experts launch
+_MAX_PREFILL_PAIRS = 65536  # SLUICE_MAX_PREFILL_PAIRS
+_MAX_PREFILL_WORKSPACE = 1 << 30  # bytes; larger chunks run in slices
 
 
 def _stream(device: torch.device) -> int:
@@ -118,6 +120,11 @@ class _Workspace:
             self.buf[idx] = cur
         return cur
 
+    def size(self, device: torch.device) -> int:
+        idx = device.index if device.index is not None else torch.cuda.current_device()
+        cur = self.buf.get(idx)
+        return 0 if cur is None else cur.numel()
+
 
 _WS = _Workspace()
 
@@ -192,47 +199,74 @@ def _fused_experts_impl(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch
             raise ValueError(f"plan must be a contiguous int32 buffer of >= "
                              f"{lib.sluice_moe_plan_ints(T, k)} ints on {x.device} "
                              f"(T={T}, k={k}, at most {chunk} tokens)")
-    if T > chunk:
-        # more (token, expert) pairs than one launch takes (a prefill chunk on
-        # the classic path): tokens are independent, so run slices of them
-        for t0 in range(0, T, chunk):
-            t1 = min(T, t0 + chunk)
-            out[t0:t1] = _fused_experts_impl(
-                x[t0:t1], w1, w2, tw[t0:t1], ids[t0:t1], activation, global_num_experts,
-                expert_map, w1_scale, w2_scale, block_shape, routed_scaling_factor,
-                None if shared_output is None else shared_output[t0:t1], shared_w1, shared_w2,
-                shared_w1_scale, shared_w2_scale)
-        return out
-    nbytes = workspace_bytes(T, H, I, k, Is)
-    ws = _WS.get(x.device, nbytes)
     sh = None
     if shared_output is not None:
         sh = shared_output.contiguous()
         if sh.dtype != torch.bfloat16 or sh.shape != x.shape:
             raise ValueError("shared_output must be bf16 [T, H]")
-    stream = _stream(x.device)
-    if w1.dtype == torch.bfloat16:
-        rc = lib.sluice_fused_experts_bf16(
-            x.data_ptr(), w1.data_ptr(), w2.data_ptr(), tw.data_ptr(), ids.data_ptr(), emap_ptr,
-            T, H, I, k, E, S, float(routed_scaling_factor), _ptr(shared_w1), _ptr(shared_w2), Is,
-            _ptr(sh), ws.data_ptr(), ws.numel(), out.data_ptr(), _ptr(plan), stream)
-        _lib.check(rc, "sluice_fused_experts_bf16")
-    elif w1.dtype in (torch.uint8, torch.float8_e4m3fn):
+    fp8 = w1.dtype in (torch.uint8, torch.float8_e4m3fn)
+    if fp8:
         if w1_scale is None or w2_scale is None:
             raise ValueError("fp8 experts need w1_scale and w2_scale")
         bn, bk = (block_shape or [128, 128])[:2]
         if Is and (shared_w1_scale is None or shared_w2_scale is None):
             raise ValueError("fp8 shared experts need shared_w1_scale and shared_w2_scale")
-        rc = lib.sluice_fused_experts_fp8(
-            x.data_ptr(), w1.data_ptr(), w1_scale.data_ptr(), w2.data_ptr(), w2_scale.data_ptr(),
-            int(bn), int(bk), tw.data_ptr(), ids.data_ptr(), emap_ptr, T, H, I, k, E, S,
-            float(routed_scaling_factor), _ptr(shared_w1), _ptr(shared_w1_scale),
-            _ptr(shared_w2), _ptr(shared_w2_scale), Is, _ptr(sh), ws.data_ptr(), ws.numel(),
-            out.data_ptr(), _ptr(plan), stream)
-        _lib.check(rc, "sluice_fused_experts_fp8")
-    else:
+    elif w1.dtype != torch.bfloat16:
         raise TypeError(f"unsupported expert dtype {w1.dtype}")
+    stream = _stream(x.device)
+    # More (token, expert) pairs than one launch takes (a prefill chunk on the
+    # classic path): tokens are independent, so run slices of them, as few as
+    # the prefill entry's bounds allow.
+    step = T if T <= chunk else _prefill_slice(T, H, I, k, Is, chunk, x.device)
+    ws = _WS.get(x.device, workspace_bytes(min(T, step), H, I, k, Is))
+    for t0 in range(0, T, step):
+        n = min(step, T - t0)
+        row = 2 * H * t0
+        xp, op = x.data_ptr() + row, out.data_ptr() + row
+        shp = None if sh is None else sh.data_ptr() + row
+        twp, idp = tw.data_ptr() + 4 * k * t0, ids.data_ptr() + 4 * k * t0
+        if n > chunk and (not fp8 or (bn == 128 and bk == 128)):
+            rc = lib.sluice_fused_experts_prefill(
+                xp, w1.data_ptr(), _ptr(w1_scale) if fp8 else None, w2.data_ptr(),
+                _ptr(w2_scale) if fp8 else None, twp, idp, emap_ptr, n, H, I, k, E, S,
+                float(routed_scaling_factor), _ptr(shared_w1), _ptr(shared_w1_scale),
+                _ptr(shared_w2), _ptr(shared_w2_scale), Is, shp, ws.data_ptr(), ws.numel(), op,
+                stream)
+            _lib.check(rc, "sluice_fused_experts_prefill")
+        elif fp8:
+            rc = lib.sluice_fused_experts_fp8(
+                xp, w1.data_ptr(), w1_scale.data_ptr(), w2.data_ptr(), w2_scale.data_ptr(),
+                int(bn), int(bk), twp, idp, emap_ptr, n, H, I, k, E, S,
+                float(routed_scaling_factor), _ptr(shared_w1), _ptr(shared_w1_scale),
+                _ptr(shared_w2), _ptr(shared_w2_scale), Is, shp, ws.data_ptr(), ws.numel(), op,
+                _ptr(plan), stream)
+            _lib.check(rc, "sluice_fused_experts_fp8")
+        else:
+            rc = lib.sluice_fused_experts_bf16(
+                xp, w1.data_ptr(), w2.data_ptr(), twp, idp, emap_ptr, n, H, I, k, E, S,
+                float(routed_scaling_factor), _ptr(shared_w1), _ptr(shared_w2), Is, shp,
+                ws.data_ptr(), ws.numel(), op, _ptr(plan), stream)
+            _lib.check(rc, "sluice_fused_experts_bf16")
     return out
+
+
+def _prefill_slice(T: int, H: int, I: int, k: int, Is: int, chunk: int, device) -> int:
+    """Tokens per launch of a call of more than ``chunk`` tokens: equal slices
+    within the prefill entry's pair and workspace bounds, or ``chunk`` where
+    the workspace cannot grow to that: while a graph is being captured, or
+    without the memory for it."""
+    per = workspace_bytes(_MAX_PAIRS, H, I, k, Is) // _MAX_PAIRS + 1
+    most = max(chunk, min(_MAX_PREFILL_PAIRS // (k + Is // I), _MAX_PREFILL_WORKSPACE // per))
+    step = -(-T // -(-T // most))
+    need = workspace_bytes(step, H, I, k, Is)
+    if _WS.size(device) < need:
+        if torch.cuda.is_current_stream_capturing():
+            return chunk
+        try:
+            _WS.get(device, need)
+        except torch.OutOfMemoryError:
+            return chunk
+    return step
 
 
 @torch.library.custom_op("sluice::fused_experts", mutates_args=())

@@ -377,3 +377,156 @@ def test_fp8_decode_all_bytes_exact():
     want = g / (1 + np.exp(-g))
     got = out.float().cpu().numpy()[0]
     np.testing.assert_allclose(got, want, rtol=8e-3, atol=1e-30)
+
+
+def _tile_case(T, H, I, Is, E, S, k, frac, fp8, seed):
+    """Device inputs of a fused_experts call: (args, kwargs)."""
+    rng = np.random.default_rng(seed)
+    g = torch.Generator(device=DEV).manual_seed(seed)
+
+    def weights(shape):
+        w = torch.randn(shape, generator=g, device=DEV)
+        if not fp8:
+            return (w * 0.02).to(torch.bfloat16), None
+        s = torch.rand((*shape[:-2], shape[-2] // 128, shape[-1] // 128), generator=g, device=DEV)
+        return (w * 0.5).to(torch.float8_e4m3fn).view(torch.uint8), s * 0.02 + 0.01
+
+    x = torch.randn((T, H), generator=g, device=DEV).to(torch.bfloat16)
+    (w13, s13), (w2, s2) = weights((S, 2 * I, H)), weights((S, H, I))
+    ids = _routing(T, E, k, rng)
+    ids[T // 2] = E + 5  # out of range: the token's pairs are not resident
+    tw = torch.from_numpy(rng.random((T, k)).astype(np.float32)).to(DEV)
+    kw = dict(global_num_experts=E, routed_scaling_factor=1.5,
+              expert_map=torch.from_numpy(_emap(E, S, rng, frac)).to(DEV))
+    if fp8:
+        kw.update(w1_scale=s13, w2_scale=s2, block_shape=[128, 128])
+    if Is:
+        (kw["shared_w1"], a), (kw["shared_w2"], b) = weights((2 * Is, H)), weights((H, Is))
+        if fp8:
+            kw.update(shared_w1_scale=a, shared_w2_scale=b)
+    return [x, w13, w2, tw, torch.from_numpy(ids).to(DEV)], kw
+
+
+def _in_slices(args, kw, n):
+    """The call in slices of n tokens (the decode kernels, for small n)."""
+    from sluice_amd import ops
+
+    x, w13, w2, tw, ids = args
+    return torch.cat([ops.fused_experts(x[t:t + n], w13, w2, tw[t:t + n], ids[t:t + n], **kw)
+                      for t in range(0, x.shape[0], n)])
+
+
+# Two correct products of the same bf16 inputs differ in the order of their
+# fp32 sums, so a value of the bf16 activations or outputs is at most one
+# rounding (2^-8 of it) apart.
+ONE_ROUNDING = 2.0 ** -8
+
+
+@pytest.mark.parametrize("T,H,I,Is,E,S,k,frac,fp8", [
+    (96, 1088, 448, 448, 40, 40, 5, 0.8, False),    # 12 pairs per slot: the smallest, odd sizes
+    (257, 1088, 448, 896, 64, 40, 5, 0.8, False),   # 64-pair tiles, partial ones
+    (801, 1088, 448, 0, 40, 40, 5, 1.0, False),     # 128-pair tiles
+    (1000, 1088, 448, 448, 40, 40, 5, 0.8, False),  # over 4096 pairs: one prefill call
+    (600, 64, 64, 0, 512, 512, 8, 0.9, False),      # over 4096 pairs, few per slot, one K chunk
+    (301, 2048, 1024, 0, 16, 16, 16, 1.0, False),   # every token to every expert
+    (300, 1088, 448, 448, 64, 40, 5, 0.0, False),   # nothing routed is resident
+    (150, 1152, 640, 640, 48, 48, 4, 0.8, True),    # fp8, 32-pair tiles
+    (500, 1152, 640, 640, 48, 48, 4, 1.0, True),    # fp8, 64-pair tiles
+    (1100, 1152, 640, 0, 64, 48, 4, 0.8, True),     # fp8, over 4096 pairs
+    (96, 9216, 512, 0, 40, 32, 4, 1.0, True),       # over 64 scale chunks of K
+])
+def test_tiled_product_matches_the_decode_kernels(T, H, I, Is, E, S, k, frac, fp8):
+    from sluice_amd import ops
+
+    print(f"tiles T={T} H={H} I={I} Is={Is} E={E} S={S} k={k} fp8={fp8}", flush=True)
+    args, kw = _tile_case(T, H, I, Is, E, S, k, frac, fp8, seed=T + H)
+    got = [ops.fused_experts(*args, **kw) for _ in range(2)]
+    ref = _in_slices(args, kw, 7)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], got[1])
+    err = om.rel_l2(got[0].float().cpu().numpy(), ref.float().cpu().numpy())
+    print(f"  rel_l2={err:.2e}", flush=True)
+    assert err <= ONE_ROUNDING
+
+
+def test_tiled_product_keeps_tokens_apart():
+    """A token of NaN and one of infinities change no other token's bits."""
+    from sluice_amd import ops
+
+    args, kw = _tile_case(257, 1088, 448, 448, 40, 40, 5, 1.0, False, seed=3)
+    clean = ops.fused_experts(*args, **kw)
+    args[0][13] = float("nan")
+    args[0][200] = float("inf")
+    got = ops.fused_experts(*args, **kw)
+    torch.cuda.synchronize()
+    assert torch.isnan(got[13]).any()
+    rest = [t for t in range(257) if t not in (13, 200)]
+    assert torch.equal(got[rest], clean[rest])
+
+
+def test_prefill_entry_bounds():
+    """Refused without touching the GPU: too many pairs, scales of one weight
+    only, sizes the kernels do not take."""
+    from sluice_amd import _lib
+
+    lib = _lib.load()
+    buf = torch.empty(1 << 20, dtype=torch.uint8, device=DEV)
+    p = buf.data_ptr()
+
+    def call(T, H, I, s13=None, s2=None, shared=None):
+        return lib.sluice_fused_experts_prefill(
+            p, p, s13, p, s2, p, p, None, T, H, I, 8, 64, 64, 1.0, shared, None, shared, None,
+            I if shared else 0, None, p, buf.numel(), p, None)
+
+    assert call(8193, 64, 64) == _lib.SLUICE_E_INVAL     # 65544 pairs
+    assert call(8000, 64, 64, shared=p) == _lib.SLUICE_E_INVAL
+    assert call(1024, 64, 64) == _lib.SLUICE_E_INVAL     # workspace too small
+    assert call(8, 128, 128, s13=p) == _lib.SLUICE_E_INVAL
+    assert call(8, 192, 128, s13=p, s2=p) == _lib.SLUICE_E_INVAL
+    assert call(8, 96, 64) == _lib.SLUICE_E_INVAL
+
+
+def test_prefill_slices_follow_the_reserved_workspace(monkeypatch):
+    """While a graph is captured a chunk whose workspace was not reserved runs
+    in slices that fit the one there is; the replays give the eager bits."""
+    from sluice_amd import ops
+
+    args, kw = _tile_case(1000, 1088, 448, 0, 40, 40, 5, 0.8, False, seed=5)
+    want = ops.fused_experts(*args, **kw)
+    monkeypatch.setattr(ops, "_WS", ops._Workspace())
+    ops.reserve_workspace(DEV, 819, 1088, 448, 5)  # 4095 pairs
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.fused_experts(*args, **kw)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert om.rel_l2(got.float().cpu().numpy(), want.float().cpu().numpy()) <= ONE_ROUNDING
+
+
+def test_tiled_product_over_a_map_whose_slots_streamed():
+    """A prefill call over the map of a layer whose last gap filled slots
+    waits for them like the decode kernels do, and gives their product."""
+    from sluice_amd import ops
+    from sluice_amd.decoder import SyntheticMoELayer, build_offloaded
+
+    E, S, k, H, I = 24, 16, 4, 2048, 1024
+    layer = SyntheticMoELayer(H, I, E, k, renorm=True, seed=4, device=DEV)
+    off = build_offloaded([layer], slots=S, device=DEV)
+    try:
+        g = torch.Generator(device=DEV).manual_seed(6)
+        layer(torch.randn((4, H), generator=g, device=DEV).to(torch.bfloat16))  # fills slots
+        x = torch.randn((64, H), generator=g, device=DEV).to(torch.bfloat16)
+        ids = torch.randint(0, E, (64, k), generator=g, device=DEV, dtype=torch.int32)
+        tw = torch.rand((64, k), generator=g, device=DEV)
+        args = [x, layer.w13_weight, layer.w2_weight, tw, ids]
+        kw = dict(global_num_experts=E, expert_map=layer.expert_map)
+        got = ops.fused_experts(*args, **kw)
+        ref = _in_slices(args, kw, 4)
+        torch.cuda.synchronize()
+        assert (ref != 0).any()
+        assert om.rel_l2(got.float().cpu().numpy(), ref.float().cpu().numpy()) <= ONE_ROUNDING
+    finally:
+        off.close()
