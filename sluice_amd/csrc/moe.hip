@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "plan.h"
@@ -802,13 +803,16 @@ __global__ __launch_bounds__(kThreads) void moe_gemm2_split_kernel(
 // and not added.  !SPEC (large calls: prefill chunks, classic waves, where
 // many pairs of a wave are invalid and the kernel is bandwidth-bound): the
 // valid words first, then only the valid rows.
+// topk_w: the routing weights the partials still need (the tiled product), or
+// nullptr (the decode kernels have applied them).
 constexpr int kMaxShared = 4;
 // partial bytes of a call above which the combine reads valid words first
 constexpr long kCombineCheckFirstBytes = 2L << 20;
 
 template <bool SPEC>
 __device__ __forceinline__ void combine4(const float* __restrict__ partial,
-                                         const int32_t* __restrict__ valid, int t, int T, int k,
+                                         const int32_t* __restrict__ valid,
+                                         const float* __restrict__ topk_w, int t, int T, int k,
                                          int n_sh, int H, int h, float scale,
                                          const uint16_t* __restrict__ shared,
                                          uint16_t* __restrict__ out) {
@@ -833,7 +837,7 @@ __device__ __forceinline__ void combine4(const float* __restrict__ partial,
   f32x4_t acc = zero, acs = zero;
 #pragma unroll
   for (int j = 0; j < SLUICE_MAX_TOPK; ++j)
-    if (ok[j]) acc += v[j];
+    if (ok[j]) acc += topk_w != nullptr ? topk_w[t * k + j] * v[j] : v[j];
 #pragma unroll
   for (int u = 0; u < kMaxShared; ++u)
     if (u < n_sh) acs += vs[u];
@@ -850,13 +854,14 @@ __device__ __forceinline__ void combine4(const float* __restrict__ partial,
 
 template <bool SPEC>
 __global__ __launch_bounds__(256) void moe_combine_kernel(
-    const float* __restrict__ partial, const int32_t* __restrict__ valid, int T, int k, int n_sh,
-    int H, float scale, const uint16_t* __restrict__ shared, uint16_t* __restrict__ out) {
+    const float* __restrict__ partial, const int32_t* __restrict__ valid,
+    const float* __restrict__ topk_w, int T, int k, int n_sh, int H, float scale,
+    const uint16_t* __restrict__ shared, uint16_t* __restrict__ out) {
   const int t = blockIdx.y;
   const int h = (blockIdx.x * 256 + threadIdx.x) * 4;
   if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) SLUICE_DTRACE(13, T);
   if (h >= H) return;
-  combine4<SPEC>(partial, valid, t, T, k, n_sh, H, h, scale, shared, out);
+  combine4<SPEC>(partial, valid, topk_w, t, T, k, n_sh, H, h, scale, shared, out);
 }
 
 #include "tile.h"
@@ -967,53 +972,52 @@ int check_common(int T, int H, int I, int k, int E, int S, int n_sh, const void*
   return SLUICE_OK;
 }
 
-int launch_combine(const float* partial, const int32_t* valid, int T, int k, int n_sh, int H,
-                   float scale, const void* shared, void* out, hipStream_t st) {
+int launch_combine(const float* partial, const int32_t* valid, const float* topk_w, int T, int k,
+                   int n_sh, int H, float scale, const void* shared, void* out, hipStream_t st) {
   dim3 grid((H / 4 + 255) / 256, T);
   if ((long)T * k * H * (long)sizeof(float) > kCombineCheckFirstBytes)
-    hipLaunchKernelGGL(moe_combine_kernel<false>, grid, dim3(256), 0, st, partial, valid, T, k,
-                       n_sh, H, scale, (const uint16_t*)shared, (uint16_t*)out);
+    hipLaunchKernelGGL(moe_combine_kernel<false>, grid, dim3(256), 0, st, partial, valid,
+                       topk_w, T, k, n_sh, H, scale, (const uint16_t*)shared, (uint16_t*)out);
   else
-    hipLaunchKernelGGL(moe_combine_kernel<true>, grid, dim3(256), 0, st, partial, valid, T, k,
-                       n_sh, H, scale, (const uint16_t*)shared, (uint16_t*)out);
+    hipLaunchKernelGGL(moe_combine_kernel<true>, grid, dim3(256), 0, st, partial, valid,
+                       topk_w, T, k, n_sh, H, scale, (const uint16_t*)shared, (uint16_t*)out);
   return (int)hipGetLastError();
 }
 
-// Tile shapes: 128 weight rows x BM pairs, four waves of 32 rows each.  As
-// many stages as let two workgroups share a CU's LDS; two independent
-// workgroups hide each other's barriers (one 8-wave workgroup of 256 rows
-// measured the same or slower: 372-428 against 338-395 us for gemm1 at 4096
-// tokens of the Qwen3 shape).
+// Tile shapes.  While the weights bound the call (64 pairs and fewer per
+// tile), 128 weight rows per four-wave workgroup and stages that let two
+// workgroups share a CU; beyond, one eight-wave workgroup of 256 rows, which
+// reads the tokens half as often (gemm1 at 4096 tokens of the Qwen3 shape:
+// 306 us against 325 for 128 x 128 tiles, 386 for 128 x 64).
 template <bool FP8, bool G1, int BM>
 struct TileFor {
-  using type = TileCfg<FP8, G1, 128, BM, 4, 1, BM == 128 ? 2 : FP8 ? (BM == 64 ? 2 : 3)
-                                                                   : (BM == 64 ? 3 : 4)>;
+  using type = TileCfg<FP8, G1, 128, BM, 4, 1, FP8 && BM == 64 ? 2 : 3>;
 };
-template <>
-struct TileFor<false, false, 128> {  // short K (I): 219 against 238 us
-  using type = TileCfg<false, false, 256, 128, 4, 2, 3>;
+template <bool G1>
+struct TileFor<false, G1, 128> {
+  using type = TileCfg<false, G1, 256, 128, 8, 1, 3>;
 };
 
 // Pairs per tile, or 0 for the decode kernels, from the mean pairs per slot.
 // The decode kernels read an expert's weights once per 16 of its tokens and
-// so win while most experts have one block; at 12 pairs per slot the tiles
-// took over (us, decode kernels / tiles: V2-Lite 48 slots 177 / 187 at 12
-// with even routing and 207 / 188 with Zipf, 204 / 186 at 16; Qwen3 256 /
-// 246 at 12; V3 fp8 610 / 586 at 8, 701 / 612 at 12).  Larger tiles reuse
-// the weights more and pad more: 32 / 64 / 128 pairs gave 186 / 195 / 234 at
-// 16 per slot, 255 / 215 / 246 at 64, 385 / 289 / 267 at 128 (V2-Lite).
+// so win while most experts have one block.  Whole calls in us, decode
+// kernels / tiles, even and Zipf routing: V2-Lite over 48 slots 161 / 176 and
+// 176 / 180 at 8 pairs per slot, 177 / 175 and 207 / 174 at 12; Qwen3 222 /
+// 225 and 187 / 161 at 8, 256 / 229 and 243 / 178 at 12; V3 fp8 422 / 449 at
+// 4, 610 / 559 at 8.  Larger tiles reuse the weights more and pad more: 64 /
+// 128 pairs gave 246 / 249 at 32 per slot and 300 / 279 at 64 (Qwen3), 287 /
+// 244 at 128 (V2-Lite); fp8 32 / 64 pairs 592 / 637 at 16, 672 / 657 at 24.
 //
 // A call over few slots must also fill the device: the tiles are taken where
 // they make at least one item per CU.
 template <bool FP8>
 int tile_pairs(const CallShape& cs, int E, int S) {
   const int slots = std::min(E, S), P = cs.T * cs.k;
-  if (P > SLUICE_MAX_PAIRS || P >= 12 * slots) {
-    const int bm = FP8 ? (P < 32 * slots ? 32 : 64) : P < 20 * slots ? 32 : P < 100 * slots ? 64 : 128;
-    const long items = (long)std::max(P / bm, slots) * std::min(cs.I / 64, cs.H / 128);
-    if (P > SLUICE_MAX_PAIRS || items >= 256) return bm;
-  }
-  return 0;
+  if (P <= SLUICE_MAX_PAIRS && P < (FP8 ? 6 : 10) * slots) return 0;
+  const int bm = FP8 ? (P < 20 * slots ? 32 : 64) : P < 64 * slots ? 64 : 128;
+  const int rows = bm == 128 ? 256 : 128;
+  const long items = (long)std::max(P / bm, slots) * std::min(2 * cs.I / rows, cs.H / rows);
+  return P > SLUICE_MAX_PAIRS || items >= 256 ? bm : 0;
 }
 
 // Workgroups of a persistent tile launch: as many as fit the device at once
@@ -1055,9 +1059,9 @@ int run_tiles(const TileArgs& a, long tiles, hipStream_t st) {
 }
 
 // The tiled product: sort, gemm1, gemm2, combine.  The sorted call sits in
-// the workspace's plan area, which is always larger: the records, order and
-// flags take at most 7 ints per pair (+ 2048 for the slots' partial tiles,
-// when P > SLUICE_MAX_PAIRS), the plan 19.
+// the workspace's plan area, which is always larger (checked): with up to 4
+// shared groups the records, order and flags take at most 5 ints per pair
+// and 24 more, the plan 19 per pair and 4, and a tiled call has 12 pairs.
 template <bool FP8>
 int run_tiled(const void* x, const ExpertW& W, const float* tw, const int32_t* ti,
               const int32_t* map, const CallShape& cs, int E, int S, int n_sh, int bm, float scale,
@@ -1067,22 +1071,20 @@ int run_tiled(const void* x, const ExpertW& W, const float* tw, const int32_t* t
   TilePlan pl;
   pl.hdr = w.plan;
   pl.tiles = (TileRec*)(w.plan + kPlanHeader);
-  pl.order = (int32_t*)(pl.tiles + tiles);
-  pl.valid = pl.order + P2;
-  if ((size_t)(pl.valid + P - w.plan) > plan_ints(P)) return SLUICE_E_INVAL;
-  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(kSortThreads), 0, st, ti, P, map, E, S,
-                     W.wait.pending, T, n_sh, bm, pl);
+  pl.valid = (int32_t*)(pl.tiles + tiles);
+  pl.order = (uint16_t*)(pl.valid + (P + 3) / 4 * 4);
+  if ((size_t)(pl.order + P2 - (uint16_t*)w.plan) > 2 * plan_ints(P)) return SLUICE_E_INVAL;
+  auto sort = P <= 8 * kSortThreads ? moe_sort_kernel<8> : moe_sort_kernel<64>;
+  static_assert(SLUICE_MAX_PREFILL_PAIRS <= 64 * kSortThreads, "sort registers");
+  hipLaunchKernelGGL(sort, dim3(1), dim3(kSortThreads), 0, st, ti, P, map, E, S, W.wait.pending, T,
+                     n_sh, bm, pl);
   SLUICE_HIP_CHECK(hipGetLastError());
-  const TileArgs a{(const uint16_t*)x, W, pl, cs, tw, w.act, w.partial};
-  int rc = SLUICE_OK;
-  if (bm == 32)
-    rc = run_tiles<FP8, 32>(a, tiles, st);
-  else if (FP8 || bm == 64)
-    rc = run_tiles<FP8, 64>(a, tiles, st);
-  else
-    rc = run_tiles<FP8, FP8 ? 64 : 128>(a, tiles, st);
+  const TileArgs a{(const uint16_t*)x, W, pl, cs, w.act, w.partial};
+  // fp8 tiles have 32 or 64 pairs, bf16 ones 64 or 128
+  const int rc = bm == 64 ? run_tiles<FP8, 64>(a, tiles, st)
+                          : run_tiles<FP8, (FP8 ? 32 : 128)>(a, tiles, st);
   if (rc != SLUICE_OK) return rc;
-  return launch_combine(w.partial, pl.valid, T, cs.k, n_sh, cs.H, scale, shared, out, st);
+  return launch_combine(w.partial, pl.valid, tw, T, cs.k, n_sh, cs.H, scale, shared, out, st);
 }
 
 // plan: a plan of these ids over this map built on the stream before the
@@ -1140,8 +1142,8 @@ int run_experts(const void* x, const ExpertW& W, const float* tw, const int32_t*
                        tw, cs, w.partial);
     SLUICE_HIP_CHECK(hipGetLastError());
   }
-  return launch_combine(w.partial, plan + kPlanHeader + (size_t)kBlockInts * P, T, k, n_sh, H,
-                        scale, shared, out, st);
+  return launch_combine(w.partial, plan + kPlanHeader + (size_t)kBlockInts * P, nullptr, T, k,
+                        n_sh, H, scale, shared, out, st);
 }
 
 // Shared-expert weights: none (shared_I == 0), or n_sh = shared_I / I
@@ -1361,8 +1363,8 @@ extern "C" int sluice_moe_combine(const float* partial, const int32_t* plan, int
   if (T <= 0 || k <= 0 || H <= 0 || H % 4 || (long)T * k > SLUICE_MAX_PAIRS || !partial || !plan ||
       !out || (((uintptr_t)shared | (uintptr_t)out | (uintptr_t)partial) & 7))
     return SLUICE_E_INVAL;
-  return launch_combine(partial, plan + kPlanHeader + (size_t)kBlockInts * T * k, T, k, 0, H, scale,
-                        shared, out, (hipStream_t)stream);
+  return launch_combine(partial, plan + kPlanHeader + (size_t)kBlockInts * T * k, nullptr, T, k, 0,
+                        H, scale, shared, out, (hipStream_t)stream);
 }
 
 // Gap timeline tracing (trace.h): this translation unit's ring.

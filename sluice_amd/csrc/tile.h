@@ -13,20 +13,26 @@
 //   * gemm1: act[pos] = bf16(silu(g) * u), rows in sorted order, so that
 //     gemm2 reads them without a gather; a wave holds gate and up rows of the
 //     same channels.
-//   * gemm2: partial[pair] = w * W2 . act[pos] (fp32), which the combine sums
-//     as it does for the decode kernels.
+//   * gemm2: partial[pair] = W2 . act[pos] (fp32), which the combine weights
+//     and sums.
 //
-// Bound: HBM while the experts have few tokens (the weights are read once),
-// the matrix cores and the LDS operand reads beyond.  Whole calls against the
-// decode kernels: Qwen3 shape, 4096 tokens, 4084 -> 618 us; V2-Lite shape,
-// 509 tokens over 48 slots, 628 -> 233 us; V3 fp8, 384 tokens over 64 of 256
-// experts, 1364 -> 794 us.
+// Bound: HBM while the experts have few tokens (the weights are read once;
+// 4.9 TB/s in gemm1 of the V2-Lite call below, the DMA stream alone reaches
+// 6.2), the operand traffic out of L2 beyond (a 4096-token call runs no faster
+// with the LDS reads scheduled between the products).  Whole calls against the
+// decode kernels: Qwen3 shape, 4096 tokens, 4084 -> 570 us; V2-Lite
+// shape, 509 tokens over 48 slots, 628 -> 229 us; V3 fp8, 384 tokens over 64 of
+// 256 experts, 1364 -> 725 us.
 //
 // LDS rows are 128 bytes (64 bf16 or 128 fp8 of K) in eight 16-byte
-// segments, segment s of row r at s ^ (r & 7), so the row-major DMA writes
-// and the MFMA-order reads are both free of bank conflicts; the swizzle is
-// in the lanes' global addresses, since a DMA writes its lanes consecutively.
-// The K order inside a chunk is the same permutation for both operands.
+// segments, segment s of row r at s ^ (r & 7); the swizzle is in the lanes'
+// global addresses, since a DMA writes its lanes consecutively.  A 16-byte
+// LDS read serves 16 lanes at a time over 64 banks, and the lanes that meet
+// come from two neighbouring K groups (lanes 0-3, 12-15 and 20-27, ...): the
+// K groups of one read take neighbouring segments (4m + kb), so that the two
+// groups fall on even and odd segments (with segments 2kb + m half of the
+// LDS cycles were conflicts).  The fp8 product's token segments are stored in
+// the order its 16-value weight segments take them.
 //
 // (Internal to moe.hip, which includes it inside its anonymous namespace.)
 #pragma once
@@ -43,14 +49,21 @@ static_assert(sizeof(TileRec) == 16, "TileRec");
 
 // The sorted call: header {tiles, 0, 0, 0}, then the tile records.
 struct TilePlan {
-  int32_t* hdr;
+  int32_t* hdr;    // {tiles, routed tiles, 0, 0}
   TileRec* tiles;
-  int32_t* order;  // [P2]
-  int32_t* valid;  // [P]
+  uint16_t* order;  // [P2] pair of a sorted position
+  int32_t* valid;   // [P]
 };
+static_assert(SLUICE_MAX_PREFILL_PAIRS <= 65536, "pairs are 16-bit");
 
 constexpr int kSortThreads = 1024;
 constexpr int kSortWaves = kSortThreads / SLUICE_WAVE;
+
+// Pairs per tile of a slot with n > 0 of them.
+__host__ __device__ inline int tile_size(int n, int bm) {
+  const int nt = (n + bm - 1) / bm;
+  return ((n + nt - 1) / nt + 15) & ~15;
+}
 
 // Upper bound of the tiles of a call over at most `slots` slots.
 inline long tile_bound(int P, int slots, int T, int n_sh, int bm) {
@@ -58,16 +71,26 @@ inline long tile_bound(int P, int slots, int T, int n_sh, int bm) {
 }
 
 // Pairs grouped by slot (resident slots ascending, then those whose rows may
-// still stream), cut into tiles of bm pairs.  The order of the pairs inside a
-// slot is whatever the LDS atomics make it: a pair's product does not depend
-// on its column.
+// still stream), cut into tiles of at most bm pairs.  The order of the pairs
+// inside a slot is whatever the LDS atomics make it: a pair's product does
+// not depend on its column.  One workgroup, latency-bound: a thread keeps its
+// U pairs' slots and ranks in registers between counting and placing, and the
+// pairs are placed in LDS and written out whole (scattered global stores,
+// one line each, took most of the kernel).  P <= U * kSortThreads.
+template <int U>
 __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     const int32_t* __restrict__ ids, int P, const int32_t* __restrict__ map, int E, int S,
     const int32_t* __restrict__ pending, int T, int n_sh, int bm, TilePlan pl) {
   __shared__ int slot_of[SLUICE_MAX_EXPERTS];
-  __shared__ int cnt[SLUICE_MAX_SLOTS], cur[SLUICE_MAX_SLOTS];
+  __shared__ int cnt[SLUICE_MAX_SLOTS];
   __shared__ int wsum[4][kSortWaves];
+  __shared__ __align__(16) uint16_t placed[U * kSortThreads];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int B = 8;  // ids in flight per thread
+  static_assert(U % B == 0, "sort batches");
+  int at[U];  // slot | rank << 10, -1 = not resident
+#pragma unroll
+  for (int u = 0; u < B; ++u) at[u] = tid + u * kSortThreads < P ? ids[tid + u * kSortThreads] : -1;
   for (int e = tid; e < E; e += kSortThreads) {
     const int s = map != nullptr ? map[e] : e;
     slot_of[e] = (unsigned)s < (unsigned)S ? s : -1;
@@ -75,26 +98,28 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
   for (int s = tid; s < S; s += kSortThreads) cnt[s] = 0;
   const int pend = tid < S && pending != nullptr && pending[tid] != 0 ? 1 : 0;
   __syncthreads();
-  constexpr int U = 8;  // ids in flight per thread
-  for (int p0 = tid; p0 < P; p0 += U * kSortThreads) {
-    int g[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int p = p0 + u * kSortThreads;
-      g[u] = p < P ? ids[p] : -1;
+  for (int b = 0; b < U; b += B) {
+    if (b * kSortThreads >= P) break;
+    if (b + B < U) {
+#pragma unroll
+      for (int u = b + B; u < b + 2 * B; ++u)
+        at[u] = tid + u * kSortThreads < P ? ids[tid + u * kSortThreads] : -1;
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int p = p0 + u * kSortThreads;
-      const int s = (unsigned)g[u] < (unsigned)E ? slot_of[g[u]] : -1;
-      if (s >= 0) atomicAdd(&cnt[s], 1);
+    for (int u = b; u < b + B; ++u) {
+      const int p = tid + u * kSortThreads;
+      const int s = (unsigned)at[u] < (unsigned)E ? slot_of[at[u]] : -1;
+      at[u] = s >= 0 ? s | atomicAdd(&cnt[s], 1) << 10 : -1;
       if (p < P) pl.valid[p] = s >= 0 ? 1 : 0;
     }
   }
   __syncthreads();
   // Exclusive scans over the slots (thread s owns slot s): pairs and tiles,
   // the resident slots' and the pending ones'.
-  const int n = tid < S ? cnt[tid] : 0, nt = (n + bm - 1) / bm;
+  const int n = tid < S ? cnt[tid] : 0;
+  // Equal tiles, whole fragments of 16: ceil(n / bm) of them, or fewer.
+  const int size = n > 0 ? tile_size(n, bm) : 16, nt = (n + size - 1) / size;
   int v[4] = {pend ? 0 : n, pend ? 0 : nt, pend ? n : 0, pend ? nt : 0}, in[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
@@ -117,34 +142,33 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
   const int o = pend ? 2 : 0;
   const int pos = (pend ? tot[0] : 0) + base[o] + in[o] - v[o];
   const int ft = (pend ? tot[1] : 0) + base[o + 1] + in[o + 1] - v[o + 1];
-  if (tid < S) {
-    cur[tid] = pos;
-    for (int i = 0; i < nt; ++i)
-      pl.tiles[ft + i] = TileRec{tid | (pend ? kPendingBit : 0), pos + i * bm,
-                                 min(bm, n - i * bm), (uint32_t)ft | ((uint32_t)nt << 16)};
+  if (tid < S) cnt[tid] = pos;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u * kSortThreads >= P) break;
+    if (tid + u * kSortThreads < P && at[u] >= 0)
+      placed[cnt[at[u] & 1023] + (at[u] >> 10)] = (uint16_t)(tid + u * kSortThreads);
   }
-  const int routed = tot[1] + tot[3], per = (T + bm - 1) / bm;
+  for (int i = 0; i < nt; ++i)  // 0 beyond the slots
+    pl.tiles[ft + i] = TileRec{tid | (pend ? kPendingBit : 0), pos + i * size,
+                               min(size, n - i * size), (uint32_t)ft | ((uint32_t)nt << 16)};
+  const int routed = tot[1] + tot[3], ssize = tile_size(T, bm), per = (T + ssize - 1) / ssize;
   for (int i = tid; i < n_sh * per; i += kSortThreads) {
     const int g = i / per, c = i - g * per;
-    pl.tiles[routed + i] = TileRec{S + g, P + g * T + c * bm, min(bm, T - c * bm),
+    pl.tiles[routed + i] = TileRec{S + g, P + g * T + c * ssize, min(ssize, T - c * ssize),
                                    (uint32_t)(routed + g * per) | ((uint32_t)per << 16)};
   }
-  for (int i = tid; i < n_sh * T; i += kSortThreads) pl.order[P + i] = P + i;
-  if (tid == 0) pl.hdr[0] = routed + n_sh * per;
-  __syncthreads();
-  for (int p0 = tid; p0 < P; p0 += U * kSortThreads) {
-    int g[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int p = p0 + u * kSortThreads;
-      g[u] = p < P ? ids[p] : -1;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int s = (unsigned)g[u] < (unsigned)E ? slot_of[g[u]] : -1;
-      if (s >= 0) pl.order[atomicAdd(&cur[s], 1)] = p0 + u * kSortThreads;
-    }
+  for (int i = tid; i < n_sh * T; i += kSortThreads) pl.order[P + i] = (uint16_t)(P + i);
+  if (tid == 0) {
+    pl.hdr[0] = routed + n_sh * per;
+    pl.hdr[1] = routed;
   }
+  __syncthreads();
+  const int used = tot[0] + tot[2];
+  for (int i = tid; i < used / 8; i += kSortThreads)
+    reinterpret_cast<u32x4_t*>(pl.order)[i] = reinterpret_cast<const u32x4_t*>(placed)[i];
+  if (tid < used % 8) pl.order[used / 8 * 8 + tid] = placed[used / 8 * 8 + tid];
 }
 
 // 16 bytes per lane from base + voff into LDS at lds + 16 * lane.  No
@@ -169,10 +193,23 @@ struct TileArgs {
   ExpertW W;
   TilePlan plan;
   CallShape cs;
-  const float* topk_w;
   uint16_t* act;
   float* partial;
 };
+
+// A uniform load of what an earlier kernel wrote, through the scalar cache
+// (the compiler takes a vector load past the DMA's memory clobbers).
+template <typename T>
+__device__ __forceinline__ T ldu(const T* p) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
+  struct Words {
+    uint32_t w[sizeof(T) / 4];
+  } r;
+#pragma unroll
+  for (size_t i = 0; i < sizeof(T) / 4; ++i)
+    r.w[i] = ((const __attribute__((address_space(4))) uint32_t*)(uintptr_t)p)[i];
+  return __builtin_bit_cast(T, r);
+}
 
 // CH weight rows x BM pairs per item, WC x WP waves, ST stages.
 template <bool FP8_, bool G1_, int CH_, int BM_, int WC_, int WP_, int ST_>
@@ -190,6 +227,11 @@ struct TileCfg {
   static_assert(NA * NW * 8 == CH && NB * NW * 8 == BM * SUB && FM % 2 == 0, "tile split");
 };
 
+// Persistent workgroups.  While an item's last products run, nothing of the
+// next one is known to the memory system, and its first stage is three
+// dependent loads away (record, tokens, operands): so the next item's record
+// and tokens are loaded behind the current item's first stages, and its first
+// stages are issued before the current item's epilogue.
 template <typename C>
 __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
   constexpr int CH = C::CH, BM = C::BM, NW = C::NW, FM = C::FM, FN = C::FN, ST = C::ST;
@@ -199,58 +241,92 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int wc = wave % C::WC, wp = wave / C::WC;
   const int R = lane & 15, kb = lane >> 4;
-  const int H = a.cs.H, I = a.cs.I, P = a.cs.T * a.cs.k;
+  const int H = a.cs.H, I = a.cs.I;
   const int n_out = G1 ? I : H, K = G1 ? H : I;
   const int n_cb = (n_out + C::kOut - 1) / C::kOut;
   const int nk = K / C::KS;
-  const int total = a.plan.hdr[0] * n_cb;
+  const uint32_t by_k = 0xffffffffu / (uint32_t)a.cs.k + 1;
   const uint32_t lds0 =
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
   // XCD x (workgroups are dealt to the 8 XCDs in turn) takes a contiguous
-  // eighth of the items, so the tiles and channel blocks of an expert meet
-  // in one L2.
+  // eighth of the routed items, so the tiles and channel blocks of an expert
+  // meet in one L2, and an eighth of the shared ones, whose weights serve
+  // many tiles: each XCD reads its share of the weights.
+  const int routed = ldu(a.plan.hdr + 1) * n_cb, shared = ldu(a.plan.hdr) * n_cb - routed;
   const int xcds = (int)gridDim.x % 8 == 0 ? 8 : 1;
   const int xcd = (int)blockIdx.x % xcds, rank = (int)blockIdx.x / xcds;
   const int per_xcd = (int)gridDim.x / xcds;
-  const int i_end = (int)((long)total * (xcd + 1) / xcds);
+  const int r0 = (int)((long)routed * xcd / xcds), rn = (int)((long)routed * (xcd + 1) / xcds) - r0;
+  const int s0 = (int)((long)shared * xcd / xcds), sn = (int)((long)shared * (xcd + 1) / xcds) - s0;
   const int seg = (lane & 7) ^ (lane >> 3);
-  for (int item = (int)((long)total * xcd / xcds) + rank; item < i_end; item += per_xcd) {
-    const TileRec r0 = a.plan.tiles[item / n_cb];
-    const int ft = (int)(r0.ft_nt & 0xffff), nt = (int)(r0.ft_nt >> 16);
-    const int local = item - ft * n_cb;
-    const int cb = local / nt;
-    const TileRec rec = a.plan.tiles[ft + local - cb * nt];
-    const int slot = __builtin_amdgcn_readfirstlane(rec.slot_field) & kSlotMask;
-    const int pos0 = __builtin_amdgcn_readfirstlane(rec.pos0);
-    const int count = __builtin_amdgcn_readfirstlane(rec.count);
-    const int ch0 = cb * C::kOut;
-    await_slot(a.W.wait, rec.slot_field);
-    // Operand addresses of this lane.
-    const uint8_t *abase, *bbase;
-    uint32_t ald;
-    const float *sc0 = nullptr, *sc1 = nullptr;  // fp8 scale rows (chunk c at [c])
-    const int wrow = G1 ? ch0 + wc * (C::CW / 2) : ch0 + wc * C::CW;  // the wave's first channel
-    const int srow = min(wrow, n_out - 1);
+  const int bseg = FP8 ? 2 * (seg & 3) + (seg >> 2) : seg;  // token segment of this lane
+
+  struct Item {
+    int slot_field, pos0, count, cb;
+  };
+  // The n-th item of this XCD (the caller checks n < rn + sn).
+  auto item_at = [&](int n) {
+    const int item = n < rn ? r0 + n : routed + s0 + (n - rn);
+    const TileRec t = ldu(a.plan.tiles + item / n_cb);
+    const int ft = (int)(t.ft_nt & 0xffff), nt = (int)(t.ft_nt >> 16);
+    const int local = item - ft * n_cb, cb = local / nt;
+    const TileRec rec = ldu(a.plan.tiles + ft + (local - cb * nt));
+    return Item{rec.slot_field, rec.pos0, rec.count, cb};
+  };
+  // The rows this lane loads of an item: pairs (gemm1; turned into tokens when
+  // they are used, so that nothing waits for them here) or sorted positions.
+  auto rows_of = [&](const Item& it, int (&rows)[C::NB]) {
+#pragma unroll
+    for (int i = 0; i < C::NB; ++i) {
+      const int g = (wave + i * NW) % (BM / 8);
+      const int row = min(g * 8 + (lane >> 3), it.count - 1);
+      rows[i] = G1 ? (int)a.plan.order[it.pos0 + row] : row;
+    }
+  };
+
+  // An item's first chunk: see issue.
+  auto first_chunk = [&](const Item& t) {
+    return (int)((unsigned)(3 * (t.slot_field & kSlotMask)) % (unsigned)nk);
+  };
+  // The wave's fp8 block scales of an item, the 64 chunks of window w, chunk
+  // c in lane c & 63 (a load per chunk would wait for every DMA in flight):
+  // of its gate and up rows, or of its hidden rows.
+  struct Scales {
+    float a, b;
+  };
+  auto scales_of = [&](const Item& t, int w) {
+    const int slot = t.slot_field & kSlotMask;
+    // a channel of the wave's 128-row blocks
+    const int ch = min(t.cb * C::kOut + wc * (G1 ? C::CW / 2 : C::CW), n_out - 1);
+    const int c = min(w * 64 + lane, nk - 1);
     if (G1) {
-      const bool routed = slot < a.W.S;
-      const size_t v = (size_t)(routed ? 0 : slot - a.W.S) * I;
-      abase = routed ? a.W.w13 + (size_t)slot * 2 * I * H * C::ESZ : a.W.sh_w13 + v * H * C::ESZ;
+      const G1Src src = g1_src<1>(a.W, a.cs, slot, ch / 16);
+      return Scales{src.sg[c], src.su[c]};
+    }
+    const float v = g2_src<1>(a.W, a.cs, slot, ch / 32).sr[c];
+    return Scales{v, v};
+  };
+
+  // Operand addresses of the item being loaded.
+  const uint8_t *abase = nullptr, *bbase = nullptr;
+  uint32_t va[C::NA], vb[C::NB];
+  int k0 = 0;
+  auto address = [&](const Item& it, const int (&rows)[C::NB]) {
+    const int slot = it.slot_field & kSlotMask, ch0 = it.cb * C::kOut;
+    uint32_t ald;
+    if (G1) {
+      const bool rt = slot < a.W.S;
+      const size_t v = (size_t)(rt ? 0 : slot - a.W.S) * I;
+      abase = rt ? a.W.w13 + (size_t)slot * 2 * I * H * C::ESZ : a.W.sh_w13 + v * H * C::ESZ;
       ald = (uint32_t)H * C::ESZ;
       bbase = (const uint8_t*)a.x;
-      if (FP8) {
-        const G1Src src = g1_src<1>(a.W, a.cs, slot, srow / 16);
-        sc0 = src.sg;
-        sc1 = src.su;
-      }
     } else {
       const G2Src src = g2_src<C::ESZ>(a.W, a.cs, slot, 0);
       abase = src.a0;
       ald = (uint32_t)src.ld * C::ESZ;
-      bbase = (const uint8_t*)(a.act + (size_t)pos0 * I);
-      if (FP8) sc0 = sc1 = g2_src<1>(a.W, a.cs, slot, srow / 32).sr;
+      bbase = (const uint8_t*)(a.act + (size_t)it.pos0 * I);
     }
     const uint32_t up = (uint32_t)(slot < a.W.S ? I : a.W.I_s);  // first up row after the gate's
-    uint32_t va[C::NA], vb[C::NB];
 #pragma unroll
     for (int i = 0; i < C::NA; ++i) {
       const int l = (wave + i * NW) * 8 + (lane >> 3);  // LDS row
@@ -265,108 +341,164 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < C::NB; ++i) {
-      const int q = wave + i * NW, sub = q / (BM / 8), g = q % (BM / 8);
-      const int row = min(g * 8 + (lane >> 3), count - 1);
-      const uint32_t t =
-          G1 ? (uint32_t)pair_token(a.cs, a.plan.order[pos0 + row]) : (uint32_t)row;
-      vb[i] = t * (uint32_t)(K * 2) + (uint32_t)(sub * 128 + seg * 16);
+      const int sub = (wave + i * NW) / (BM / 8);
+      uint32_t row = (uint32_t)rows[i];
+      if (G1)  // pair / k is exact: pairs are below 2^16
+        row = slot >= a.W.S      ? row - (uint32_t)(a.cs.T * a.cs.k + (slot - a.W.S) * a.cs.T)
+              : a.cs.k > 1 ? __umulhi(row, by_k)
+                           : row;
+      vb[i] = row * (uint32_t)(K * 2) + (uint32_t)(sub * 128 + bseg * 16);
     }
-    auto issue = [&](int k, int buf) {
-      const uint8_t* ap = abase + (size_t)k * 128;
-      const uint8_t* bp = bbase + (size_t)k * (C::KS * 2);
-      const uint32_t d = lds0 + (uint32_t)(buf * C::kStage) + (uint32_t)wave * 1024;
+    k0 = first_chunk(it);
+  };
+  // Chunk k of the item goes to stage buffer buf.  The chunks are taken from
+  // k0 on, around the end: rows are a power of two apart in many models, and
+  // workgroups that all read the same columns meet in the same memory
+  // channels.  (k0 depends on the weights alone, so a pair's sum has one
+  // order whichever tile it lands in.)
+  auto issue = [&](int k, int buf) {
+    const int kk = k + k0 < nk ? k + k0 : k + k0 - nk;
+    const uint8_t* ap = abase + (size_t)kk * 128;
+    const uint8_t* bp = bbase + (size_t)kk * (C::KS * 2);
+    const uint32_t d = lds0 + (uint32_t)(buf * C::kStage) + (uint32_t)wave * 1024;
 #pragma unroll
-      for (int i = 0; i < C::NA; ++i) dma16(d + i * NW * 1024, ap, va[i]);
+    for (int i = 0; i < C::NA; ++i) dma16(d + i * NW * 1024, ap, va[i]);
 #pragma unroll
-      for (int i = 0; i < C::NB; ++i) dma16(d + CH * 128 + i * NW * 1024, bp, vb[i]);
-    };
-    // The wave's block scales, 64 chunks at a time, chunk k in lane k & 63: a
-    // load per chunk would wait for every DMA in flight.
-    float scv0 = 0.f, scv1 = 0.f;
-    auto load_scales = [&](int k) {
-      const int c = min(k + lane, nk - 1);
-      scv0 = sc0[c];
-      scv1 = G1 ? sc1[c] : scv0;
-    };
-    if (FP8) load_scales(0);
+    for (int i = 0; i < C::NB; ++i) dma16(d + CH * 128 + i * NW * 1024, bp, vb[i]);
+  };
+  auto issue_first = [&]() {
+#pragma unroll
+    for (int s = 0; s < ST - 1; ++s)
+      if (s < nk) issue(s, s);
+  };
+
+  int n = rank;
+  if (n >= rn + sn) return;
+  Item it = item_at(n);
+  int rows[C::NB];
+  rows_of(it, rows);
+  Scales nsc = {0.f, 0.f};
+  if (FP8) nsc = scales_of(it, first_chunk(it) >> 6);
+  await_slot(a.W.wait, it.slot_field);
+  address(it, rows);
+  issue_first();
+  for (;;) {
+    const int next = n + per_xcd;
+    const bool more = next < rn + sn;
+    const Item nit = more ? item_at(next) : it;
+    rows_of(nit, rows);
+    const int kf = k0;
+    Scales sc = nsc;
+    int window = kf >> 6;
+    if (FP8) nsc = scales_of(nit, first_chunk(nit) >> 6);
+    const int count = it.count, pos0 = it.pos0, ch0 = it.cb * C::kOut;
+    const int wrow = G1 ? ch0 + wc * (C::CW / 2) : ch0 + wc * C::CW;  // the wave's first channel
+    int pair[FN];  // this lane's (gemm2), for the epilogue
+    if (!G1) {
+#pragma unroll
+      for (int g = 0; g < FN; ++g)
+        pair[g] = a.plan.order[pos0 + min((g * C::WP + wp) * 16 + R, count - 1)];
+    }
     f32x4_t acc[FM][FN];
 #pragma unroll
     for (int f = 0; f < FM; ++f)
 #pragma unroll
       for (int g = 0; g < FN; ++g) acc[f][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    dma_wait<0>();  // the previous item's readers of the stages and its stores are done
+    // The K loop over NG of the wave's FN token fragments: the fragments past
+    // the tile's pairs are left out.
+    const auto k_loop = [&](auto ng) {
+      constexpr int NG = decltype(ng)::value;
+      int buf = 0;
+      for (int k = 0; k < nk; ++k) {
+        constexpr int L = C::NA + C::NB;
+        const int ahead = min(ST - 2, nk - 1 - k);  // stages after k in flight
+        if (ST >= 4 && ahead >= 2)
+          dma_wait<(ST >= 4 ? 2 * L : 0)>();
+        else if (ST >= 3 && ahead >= 1)
+          dma_wait<(ST >= 3 ? L : 0)>();
+        else
+          dma_wait<0>();
+        if (k + ST - 1 < nk) issue(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+        const uint8_t* sa = lds + buf * C::kStage + (wc * C::CW + R) * 128;
+        const uint8_t* sb = lds + buf * C::kStage + CH * 128 + (wp * 16 + R) * 128;
+        auto ldl = [](const uint8_t* p) { return *reinterpret_cast<const u32x4_t*>(p); };
+        if constexpr (!FP8) {
 #pragma unroll
-    for (int s = 0; s < ST - 1; ++s)
-      if (s < nk) issue(s, s);
-    int buf = 0;
-    for (int k = 0; k < nk; ++k) {
-      constexpr int L = C::NA + C::NB;
-      const int ahead = min(ST - 2, nk - 1 - k);  // stages after k in flight
-      if (ST >= 4 && ahead >= 2)
-        dma_wait<(ST >= 4 ? 2 * L : 0)>();
-      else if (ST >= 3 && ahead >= 1)
-        dma_wait<(ST >= 3 ? L : 0)>();
-      else
-        dma_wait<0>();
-      if (k + ST - 1 < nk) issue(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
-      const uint8_t* sa = lds + buf * C::kStage + (wc * C::CW + R) * 128;
-      const uint8_t* sb = lds + buf * C::kStage + CH * 128 + (wp * C::PW + R) * 128;
-      auto ldl = [](const uint8_t* p) { return *reinterpret_cast<const u32x4_t*>(p); };
-      if constexpr (!FP8) {
+          for (int m = 0; m < 2; ++m) {
+            const int o = ((4 * m + kb) ^ (R & 7)) * 16;
+            u32x4_t av[FM], bv[NG];
 #pragma unroll
-        for (int m = 0; m < 2; ++m) {
-          const int o = ((2 * kb + m) ^ (R & 7)) * 16;
-          u32x4_t av[FM], bv[FN];
+            for (int f = 0; f < FM; ++f) av[f] = ldl(sa + f * 2048 + o);
 #pragma unroll
-          for (int f = 0; f < FM; ++f) av[f] = ldl(sa + f * 2048 + o);
-#pragma unroll
-          for (int g = 0; g < FN; ++g) bv[g] = ldl(sb + g * 2048 + o);
-#pragma unroll
-          for (int f = 0; f < FM; ++f)
-#pragma unroll
-            for (int g = 0; g < FN; ++g) acc[f][g] = mfma16x16x32_bf16(av[f], bv[g], acc[f][g]);
-        }
-      } else {
-        if ((k & 63) == 0 && k != 0) load_scales(k);
-        const float s0 = __uint_as_float(
-            (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(scv0), k & 63));
-        const float s1 = __uint_as_float(
-            (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(scv1), k & 63));
-        f32x4_t t[FM][FN];
-#pragma unroll
-        for (int f = 0; f < FM; ++f)
-#pragma unroll
-          for (int g = 0; g < FN; ++g) t[f][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          const int oa = ((kb + 4 * i) ^ (R & 7)) * 16;
-          u32x4_t av[FM][2];
-#pragma unroll
-          for (int f = 0; f < FM; ++f) fp8x16_to_bf16(ldl(sa + f * 2048 + oa), av[f][0], av[f][1]);
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int ob = ((2 * kb + h) ^ (R & 7)) * 16 + i * BM * 128;
-            u32x4_t bv[FN];
-#pragma unroll
-            for (int g = 0; g < FN; ++g) bv[g] = ldl(sb + g * 2048 + ob);
+            for (int g = 0; g < NG; ++g) bv[g] = ldl(sb + g * C::WP * 2048 + o);
 #pragma unroll
             for (int f = 0; f < FM; ++f)
 #pragma unroll
-              for (int g = 0; g < FN; ++g) t[f][g] = mfma16x16x32_bf16(av[f][h], bv[g], t[f][g]);
+              for (int g = 0; g < NG; ++g) acc[f][g] = mfma16x16x32_bf16(av[f], bv[g], acc[f][g]);
           }
+        } else {
+          const int kk = k + kf < nk ? k + kf : k + kf - nk;
+          if (kk >> 6 != window) {
+            window = kk >> 6;
+            sc = scales_of(it, window);
+          }
+          const float c0 = __uint_as_float(
+              (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(sc.a), kk & 63));
+          const float c1 = __uint_as_float(
+              (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(sc.b), kk & 63));
+          f32x4_t t[FM][NG];
+#pragma unroll
+          for (int f = 0; f < FM; ++f)
+#pragma unroll
+            for (int g = 0; g < NG; ++g) t[f][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            const int oa = ((4 * i + kb) ^ (R & 7)) * 16;
+            u32x4_t av[FM][2];
+#pragma unroll
+            for (int f = 0; f < FM; ++f)
+              fp8x16_to_bf16(ldl(sa + f * 2048 + oa), av[f][0], av[f][1]);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int ob = ((4 * h + kb) ^ (R & 7)) * 16 + i * BM * 128;
+              u32x4_t bv[NG];
+#pragma unroll
+              for (int g = 0; g < NG; ++g) bv[g] = ldl(sb + g * C::WP * 2048 + ob);
+#pragma unroll
+              for (int f = 0; f < FM; ++f)
+#pragma unroll
+                for (int g = 0; g < NG; ++g)
+                  t[f][g] = mfma16x16x32_bf16(av[f][h], bv[g], t[f][g]);
+            }
+          }
+#pragma unroll
+          for (int f = 0; f < FM; ++f)
+#pragma unroll
+            for (int g = 0; g < NG; ++g) acc[f][g] += (G1 && f >= FM / 2 ? c1 : c0) * t[f][g];
         }
-#pragma unroll
-        for (int f = 0; f < FM; ++f)
-#pragma unroll
-          for (int g = 0; g < FN; ++g) acc[f][g] += (G1 && f >= FM / 2 ? s1 : s0) * t[f][g];
+        buf = buf + 1 == ST ? 0 : buf + 1;
       }
-      buf = buf + 1 == ST ? 0 : buf + 1;
+    };
+    const int groups = (((count + 15) >> 4) - wp + C::WP - 1) / C::WP;  // of this wave
+    if (FN >= 4 && groups <= FN / 4)
+      k_loop(std::integral_constant<int, (FN >= 4 ? FN / 4 : FN)>{});
+    else if (groups <= FN / 2)
+      k_loop(std::integral_constant<int, FN / 2>{});
+    else if (FN >= 4 && groups <= FN * 3 / 4)
+      k_loop(std::integral_constant<int, (FN >= 4 ? FN * 3 / 4 : FN)>{});
+    else
+      k_loop(std::integral_constant<int, FN>{});
+    if (more) {
+      dma_wait<0>();  // every wave has read its last stage
+      await_slot(a.W.wait, nit.slot_field);
+      address(nit, rows);
+      issue_first();
     }
-    // Epilogue: column R of fragment g is pair pos0 + wp * PW + 16 g + R, rows
+    // Epilogue: column R of fragment g is pair pos0 + 16 (g WP + wp) + R, rows
     // 4 kb .. +4 of fragment f its channels.
 #pragma unroll
     for (int g = 0; g < FN; ++g) {
-      const int row = wp * C::PW + g * 16 + R;
+      const int row = (g * C::WP + wp) * 16 + R;
       if (row >= count) continue;
       if (G1) {
 #pragma unroll
@@ -381,17 +513,16 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
                 u32x2_t{pack2_bf16(o[0], o[1]), pack2_bf16(o[2], o[3])};
         }
       } else {
-        const int pair = a.plan.order[pos0 + row];
-        const float w = pair < P ? a.topk_w[pair] : 1.0f;
 #pragma unroll
         for (int f = 0; f < FM; ++f) {
           const int ch = wrow + f * 16 + kb * 4;
-          const f32x4_t v = acc[f][g];
           if (ch < H)
-            *reinterpret_cast<f32x4_t*>(a.partial + (size_t)pair * H + ch) =
-                f32x4_t{w * v[0], w * v[1], w * v[2], w * v[3]};
+            *reinterpret_cast<f32x4_t*>(a.partial + (size_t)pair[g] * H + ch) = acc[f][g];
         }
       }
     }
+    if (!more) return;
+    n = next;
+    it = nit;
   }
 }

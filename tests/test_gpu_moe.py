@@ -423,17 +423,18 @@ ONE_ROUNDING = 2.0 ** -8
 
 
 @pytest.mark.parametrize("T,H,I,Is,E,S,k,frac,fp8", [
-    (96, 1088, 448, 448, 40, 40, 5, 0.8, False),    # 12 pairs per slot: the smallest, odd sizes
+    (80, 1088, 448, 448, 40, 40, 5, 0.8, False),    # 10 pairs per slot: the smallest, odd sizes
     (257, 1088, 448, 896, 64, 40, 5, 0.8, False),   # 64-pair tiles, partial ones
-    (801, 1088, 448, 0, 40, 40, 5, 1.0, False),     # 128-pair tiles
+    (801, 2112, 1472, 0, 40, 40, 5, 1.0, False),    # 128-pair tiles
     (1000, 1088, 448, 448, 40, 40, 5, 0.8, False),  # over 4096 pairs: one prefill call
     (600, 64, 64, 0, 512, 512, 8, 0.9, False),      # over 4096 pairs, few per slot, one K chunk
     (301, 2048, 1024, 0, 16, 16, 16, 1.0, False),   # every token to every expert
     (300, 1088, 448, 448, 64, 40, 5, 0.0, False),   # nothing routed is resident
-    (150, 1152, 640, 640, 48, 48, 4, 0.8, True),    # fp8, 32-pair tiles
+    (72, 1152, 640, 640, 48, 48, 4, 0.8, True),     # fp8, 32-pair tiles: the smallest
     (500, 1152, 640, 640, 48, 48, 4, 1.0, True),    # fp8, 64-pair tiles
     (1100, 1152, 640, 0, 64, 48, 4, 0.8, True),     # fp8, over 4096 pairs
-    (96, 9216, 512, 0, 40, 32, 4, 1.0, True),       # over 64 scale chunks of K
+    (96, 9216, 1024, 0, 40, 32, 4, 1.0, True),      # over 64 scale chunks of K
+    (1700, 512, 256, 0, 64, 64, 5, 1.0, False),     # over 8192 pairs: the sort's larger form
 ])
 def test_tiled_product_matches_the_decode_kernels(T, H, I, Is, E, S, k, frac, fp8):
     from sluice_amd import ops
