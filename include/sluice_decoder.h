@@ -115,7 +115,7 @@ int sluice_dec_mla_decode(const void* q, int q_stride, const void* kva, int kva_
                           float scale, void* ckv_cache, void* ckvt_cache, void* kpe_cache,
                           void* work, void* out, sluice_stream_t stream);
 
-/* GQA decode with per-head q/k RMSNorm (Qwen3-MoE), one launch:
+/* GQA decode with per-head q/k RMSNorm (Qwen3-MoE):
  *   from qkv [c, (nh + 2*kvh)*hd]: q_h = rope(rmsnorm(q_h) * q_norm) (bf16),
  *   k_cache [c, kvh, L, hd] row pos[t] = bf16(rope(rmsnorm(k_g) * k_norm)),
  *   v_cache [c, kvh, L, hd] row pos[t] = v_g; then per query head h (kv head
@@ -124,7 +124,11 @@ int sluice_dec_mla_decode(const void* q, int q_stride, const void* kva, int kva_
  *   k_norm, cos_t, sin_t and the caches 16-byte aligned, out 4-byte aligned.
  *   Exactly one of qkv and qkv_parts: the QKV projection's K parts
  *   [n_parts, c, (nh + 2*kvh)*hd] fp32 (n_parts <= 4, as sluice_dec_linear_split
- *   leaves them) are summed in order and rounded to bf16 first. */
+ *   leaves them) are summed in order and rounded to bf16 first.
+ *   Caches of more than 768 rows with several query heads per kv head run
+ *   split over the rows in two launches over scratch of the library's own (26
+ *   MB per GPU, held until the process ends), calls on any streams and threads
+ *   kept apart by events; while the stream is captured, one launch. */
 int sluice_dec_gqa_decode(const void* qkv, const float* qkv_parts, int n_parts,
                           const void* q_norm, const void* k_norm,
                           const float* cos_t, const float* sin_t, const int64_t* pos, int c,

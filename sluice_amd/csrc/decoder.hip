@@ -4,11 +4,18 @@
 // model otherwise spends most of its time launching 2-5 us kernels.
 #include <math.h>
 
+#include <algorithm>
+#include <mutex>
 #include <type_traits>
 
 #include "common.h"
 #include "sluice_decoder.h"
 #include "stream.h"
+
+// Scratch of the split attention: see SplitRegion.
+constexpr int kSplitRegions = 4;
+constexpr size_t kSplitRegionBytes = 13u << 19;  // 768 splits of 16 heads' 528-byte sums
+static __device__ __align__(256) uint8_t split_scratch[kSplitRegions * kSplitRegionBytes];
 
 namespace {
 
@@ -1037,6 +1044,296 @@ __global__ __launch_bounds__(WAVES * 64) void gqa_decode_kernel(
   }
 }
 
+// The same for long caches, split over the rows, in two launches: a
+// workgroup takes one split of the rows for up to 16 query heads of one kv
+// head (a cache row is read once for all of them), the merge adds the splits
+// up.  On the matrix cores: a wave takes steps of 32 rows, scores
+// S^T[row][head] = K . q^T (two 16-row tiles, heads on N), whose registers
+// are the A operand of O[head][column] = P . V in the K order of mla_kpos;
+// V's operand (8 rows of one column per lane) is put together from 16-byte
+// row loads by byte permutes, 8 columns per lane.  P stays fp32: it enters
+// the product as three bf16 terms whose sum is P exactly.  One step's rows in
+// registers per wave and three waves per SIMD (a second step in flight at two
+// waves per SIMD measured the same).  Qwen3 heads (32 over 4), against the
+// one-launch kernel above: 36.5 -> 11.0 us for one sequence of 4000 rows, 45.6
+// -> 17.5 for 12 of 700 to 4095 (72 MB: 4.1 TB/s), 12.4 -> 9.9 for 8 of 700
+// to 1023; the second launch loses below that, 6.9 -> 8.8 for 8 of 128 to 383.
+constexpr int kSplitWaves = 4;
+constexpr int kSplitStep = 32;
+constexpr int kSplitHeads = 16;
+constexpr int kSplitMax = 16;         // splits per (token, kv head)
+constexpr int kSplitQRow = kHd + 8;   // LDS row of one head's q (padded)
+constexpr int kSplitRec = kHd + 4;    // per (split, head): max, sum, -, -, O[128]
+
+// Rows per split for n rows over `splits` of them: whole steps of every wave.
+__host__ __device__ inline int split_chunk(int n, int splits) {
+  constexpr int kRound = kSplitWaves * kSplitStep;
+  return ((n + splits - 1) / splits + kRound - 1) / kRound * kRound;
+}
+
+// grid (c * zh, kvh, splits), zh = ceil(query heads per kv head / 16).
+__global__ __launch_bounds__(kSplitWaves * 64, 3) void gqa_split_kernel(
+    const uint16_t* __restrict__ qkv, const float* __restrict__ qkv_parts, int nparts,
+    const uint16_t* __restrict__ q_norm, const uint16_t* __restrict__ k_norm,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+    const int64_t* __restrict__ pos, int nh, int kvh, int zh, int L, float eps, float scale,
+    uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache, float* __restrict__ part) {
+  __shared__ __align__(16) uint16_t qs[(kSplitHeads + 2) * kSplitQRow];  // q, then new k and v
+  __shared__ __align__(16) float om[kSplitWaves][kSplitHeads][kHd];
+  __shared__ float ms[kSplitWaves][kSplitHeads], ls[kSplitWaves][kSplitHeads];
+  const int t = blockIdx.x / zh, z = blockIdx.x - t * zh, g = blockIdx.y, tid = threadIdx.x;
+  const int splits = gridDim.z, split = blockIdx.z;
+  const long long p = pos[t];
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int R = lane & 15, kb = lane >> 4;
+  const int grp = nh / kvh, h0 = g * grp + z * kSplitHeads;
+  const int heads = min(kSplitHeads, grp - z * kSplitHeads);
+  const size_t cbase = ((size_t)t * kvh + g) * L * kHd;
+  const uint16_t* kc = k_cache + cbase;
+  const uint16_t* vc = v_cache + cbase;
+  // 16-lane group i takes vectors i and 16 + i: the query heads, then (16 and
+  // 17) the new k and v.
+  const int gi = tid >> 4, sub = tid & 15;
+  const size_t width = (size_t)(nh + 2 * kvh) * kHd;
+  auto load_vec = [&](int i) {
+    const int vec = (i < kSplitHeads ? h0 + min(i, heads - 1)
+                                     : nh + (i == kSplitHeads ? 0 : kvh) + g) * kHd + sub * 8;
+    if (qkv_parts == nullptr) return ldg16(qkv + t * width + vec);
+    // the projection's K parts: bf16(sum in part order)
+    f32x4_t a = {0.f, 0.f, 0.f, 0.f}, e = a;
+    for (int q = 0; q < nparts; ++q) {
+      const float* src = qkv_parts + ((size_t)q * (gridDim.x / zh) + t) * width + vec;
+      a += *reinterpret_cast<const f32x4_t*>(src);
+      e += *reinterpret_cast<const f32x4_t*>(src + 4);
+    }
+    return u32x4_t{pack2(a[0], a[1]), pack2(a[2], a[3]), pack2(e[0], e[1]), pack2(e[2], e[3])};
+  };
+  static_assert(kSplitWaves * 4 == kSplitHeads, "one query head per 16-lane group");
+  u32x4_t x = load_vec(gi), xn = {0u, 0u, 0u, 0u};
+  const u32x4_t wq = ldg16(q_norm + sub * 8), wk = ldg16(k_norm + sub * 8);
+  if (gi < 2) xn = load_vec(kSplitHeads + gi);
+  if (p < 0 || p >= L) return;
+  const int n = (int)p + 1, last = max((int)p - 1, 0);
+  const int chunk = split_chunk(n, splits);
+  const int r0 = split * chunk, r1 = min(n, r0 + chunk);
+  if (r0 >= n) return;
+  // A step's operands: kr[u][m] = row 16u + R, columns 8 (4m + kb); vr[j] =
+  // row (j < 4 ? 4kb + j : 16 + 4kb + j - 4), columns 8R.  (The new row is
+  // taken from LDS: the cache's may not be written yet.)
+  struct Step {
+    u32x4_t kr[2][4], vr[8];
+  };
+  auto vrow = [&](int j) { return j < 4 ? 4 * kb + j : 12 + 4 * kb + j; };
+  auto load = [&](Step& s, int b) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const uint16_t* r = kc + (size_t)min(b + 16 * u + R, last) * kHd + 8 * kb;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) s.kr[u][m] = ldg16(r + 32 * m);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      s.vr[j] = ldg16(vc + (size_t)min(b + vrow(j), last) * kHd + 8 * R);
+  };
+  Step s0;
+  const int b0 = r0 + w * kSplitStep;
+  if (b0 < r1) load(s0, b0);
+  {
+    const int ci = (int)p * 64 + (sub & 7) * 8;
+    float cs[8], sn[8], r[8];
+    *reinterpret_cast<f32x4_t*>(cs) = *reinterpret_cast<const f32x4_t*>(cos_t + ci);
+    *reinterpret_cast<f32x4_t*>(cs + 4) = *reinterpret_cast<const f32x4_t*>(cos_t + ci + 4);
+    *reinterpret_cast<f32x4_t*>(sn) = *reinterpret_cast<const f32x4_t*>(sin_t + ci);
+    *reinterpret_cast<f32x4_t*>(sn + 4) = *reinterpret_cast<const f32x4_t*>(sin_t + ci + 4);
+    auto rope = [&](u32x4_t v, u32x4_t wn) {
+      head_norm_rope(v, wn, cs, sn, eps, sub < 8, r);
+      return u32x4_t{pack2(r[0], r[1]), pack2(r[2], r[3]), pack2(r[4], r[5]), pack2(r[6], r[7])};
+    };
+    *reinterpret_cast<u32x4_t*>(&qs[gi * kSplitQRow + sub * 8]) = rope(x, wq);
+    if (gi < 2) {
+      if (gi == 0) xn = rope(xn, wk);
+      *reinterpret_cast<u32x4_t*>(&qs[(kSplitHeads + gi) * kSplitQRow + sub * 8]) = xn;
+      if (split == 0 && z == 0)
+        *reinterpret_cast<u32x4_t*>((gi == 0 ? k_cache : v_cache) + cbase + (size_t)p * kHd +
+                                    sub * 8) = xn;
+    }
+  }
+  __syncthreads();
+  u32x4_t qf[4];  // head R, columns 8 (4m + kb)
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+    qf[m] = *reinterpret_cast<const u32x4_t*>(&qs[R * kSplitQRow + 32 * m + 8 * kb]);
+  const float sl2 = scale * 1.4426950408889634f;  // scores in log2 units
+  float m = -INFINITY, l = 0.f;                    // head R's running max and sum
+  f32x4_t o[8];                                    // o[i][r]: head 4kb + r, column 8R + i
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto step = [&](Step& s, int b) {
+    if (b + kSplitStep >= n) {
+      // the last rows: the new one comes from LDS, and those past it, which
+      // hold whatever the cache held, are zeroed
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (b + 16 * u + R == n - 1)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            s.kr[u][q] = *reinterpret_cast<const u32x4_t*>(
+                &qs[kSplitHeads * kSplitQRow + 32 * q + 8 * kb]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int row = b + vrow(j);
+        if (row == n - 1)
+          s.vr[j] = *reinterpret_cast<const u32x4_t*>(&qs[(kSplitHeads + 1) * kSplitQRow + 8 * R]);
+        else if (row >= n)
+          s.vr[j] = u32x4_t{0u, 0u, 0u, 0u};
+      }
+    }
+    float pv[8];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      f32x4_t a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a = mfma16x16x32_bf16(s.kr[u][q], qf[q], a);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pv[4 * u + r] = b + 16 * u + 4 * kb + r < n ? a[r] * sl2 : -INFINITY;
+        mx = fmaxf(mx, pv[4 * u + r]);
+      }
+    }
+    const float mn = fmaxf(m, rows4_max(mx));
+    const float ref = mn == -INFINITY ? 0.f : mn;
+    const float f = __builtin_amdgcn_exp2f(m - ref);
+    float ps = 0.f;
+    u32x4_t pa[3];  // P as three bf16 terms, each the top 16 bits of what is left
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      pv[j] = __builtin_amdgcn_exp2f(pv[j] - ref);
+      ps += pv[j];
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int j = 0; j < 8; j += 2) {
+        const uint32_t a = __float_as_uint(pv[j]), e = __float_as_uint(pv[j + 1]);
+        pa[c][j / 2] = __builtin_amdgcn_perm(e, a, 0x07060302u);
+        pv[j] -= __uint_as_float(a & 0xffff0000u);
+        pv[j + 1] -= __uint_as_float(e & 0xffff0000u);
+      }
+    l = l * f + rows4_sum(ps);
+    m = mn;
+    float fr[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) fr[r] = __shfl(f, 4 * kb + r);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      u32x4_t vb;
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        vb[q] = __builtin_amdgcn_perm(s.vr[2 * q + 1][i / 2], s.vr[2 * q][i / 2],
+                                      i & 1 ? 0x07060302u : 0x05040100u);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[i][r] *= fr[r];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) o[i] = mfma16x16x32_bf16(pa[c], vb, o[i]);
+    }
+  };
+  constexpr int kRound = kSplitWaves * kSplitStep;
+  for (int b = b0; b < r1; b += kRound) {
+    step(s0, b);
+    if (b + kRound < r1) load(s0, b + kRound);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    float* dst = &om[w][4 * kb + r][8 * R];
+    *reinterpret_cast<f32x4_t*>(dst) = f32x4_t{o[0][r], o[1][r], o[2][r], o[3][r]};
+    *reinterpret_cast<f32x4_t*>(dst + 4) = f32x4_t{o[4][r], o[5][r], o[6][r], o[7][r]};
+  }
+  if (kb == 0) {
+    ms[w][R] = m;
+    ls[w][R] = l;
+  }
+  __syncthreads();
+  // the waves' states of head gi, columns 8 sub .. +8
+  if (gi < heads) {
+    float M = -INFINITY;
+#pragma unroll
+    for (int q = 0; q < kSplitWaves; ++q) M = fmaxf(M, ms[q][gi]);
+    const float ref = M == -INFINITY ? 0.f : M;
+    float den = 0.f;
+    f32x4_t a = {0.f, 0.f, 0.f, 0.f}, e = a;
+#pragma unroll
+    for (int q = 0; q < kSplitWaves; ++q) {
+      const float f = __builtin_amdgcn_exp2f(ms[q][gi] - ref);  // waves without rows: 2^-inf = 0
+      den += f * ls[q][gi];
+      a += f * *reinterpret_cast<const f32x4_t*>(&om[q][gi][8 * sub]);
+      e += f * *reinterpret_cast<const f32x4_t*>(&om[q][gi][8 * sub + 4]);
+    }
+    float* rec = part + (((size_t)t * nh + h0 + gi) * splits + split) * kSplitRec;
+    *reinterpret_cast<f32x4_t*>(rec + 4 + 8 * sub) = a;
+    *reinterpret_cast<f32x4_t*>(rec + 8 + 8 * sub) = e;
+    if (sub == 0) {
+      rec[0] = M;
+      rec[1] = den;
+    }
+  }
+}
+
+// grid (c, nh), 256 threads: 32-lane group i adds up splits i, i + 8, ... of
+// its head (four columns per lane), the groups meet in LDS.
+__global__ __launch_bounds__(kT) void gqa_merge_kernel(const float* __restrict__ part,
+                                                       const int64_t* __restrict__ pos, int nh,
+                                                       int splits, int L,
+                                                       uint16_t* __restrict__ out) {
+  __shared__ __align__(16) float acc[8][kHd];
+  __shared__ float den[8];
+  const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, i = tid >> 5, c = 4 * (tid & 31);
+  const float* rec = part + ((size_t)t * nh + h) * splits * kSplitRec;
+  const long long p = pos[t];
+  if (p < 0 || p >= L) return;
+  const int n = (int)p + 1, chunk = split_chunk(n, splits), used = (n + chunk - 1) / chunk;
+  // the first pass's loads all go out together (a split past the rows loads
+  // the first one and is not added)
+  constexpr int U = kSplitMax / 8;
+  f32x4_t v[U];
+  float m[U], l[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const float* r = rec + (size_t)(i + 8 * u < used ? i + 8 * u : 0) * kSplitRec;
+    m[u] = i + 8 * u < used ? r[0] : -INFINITY;
+    l[u] = r[1];
+    v[u] = *reinterpret_cast<const f32x4_t*>(r + 4 + c);
+  }
+  float M = -INFINITY;
+  for (int s = 0; s < used; ++s) M = fmaxf(M, rec[(size_t)s * kSplitRec]);
+  const float ref = M == -INFINITY ? 0.f : M;
+  f32x4_t a = {0.f, 0.f, 0.f, 0.f};
+  float d = 0.f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (i + 8 * u < used) {
+      const float f = __builtin_amdgcn_exp2f(m[u] - ref);
+      a += f * v[u];
+      d += f * l[u];
+    }
+  }
+  *reinterpret_cast<f32x4_t*>(&acc[i][c]) = a;
+  if (c == 0) den[i] = d;
+  __syncthreads();
+  if (tid < kHd / 2) {
+    float s = 0.f, a0 = 0.f, a1 = 0.f;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      s += den[q];
+      a0 += acc[q][2 * tid];
+      a1 += acc[q][2 * tid + 1];
+    }
+    const float inv = 1.0f / s;
+    *reinterpret_cast<uint32_t*>(out + ((size_t)t * nh + h) * kHd + 2 * tid) =
+        pack2(a0 * inv, a1 * inv);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Skinny GEMMs for decode, T <= 16 tokens, weights streamed by stream_bf16:
 //   plain: y [T, N] = x [T, K] . W [N, K]^T;
@@ -1490,6 +1787,99 @@ extern "C" int sluice_dec_mla_decode(const void* q, int q_stride, const void* kv
   return (int)hipGetLastError();
 }
 
+namespace {
+
+// Scratch of the split kernels: kSplitRegions regions per GPU, held until the
+// process ends.  A call takes a region for its two launches; the region's
+// event marks their end and the next call's stream waits for it, so calls on
+// any streams and threads are kept apart (a wait on the call's own stream
+// costs nothing on the device).  A call prefers the region its stream used
+// last, then one whose last call has ended.
+struct SplitRegion {
+  hipEvent_t done = nullptr;
+  hipStream_t last = nullptr;
+  bool used = false;
+};
+constexpr int kSplitDevices = 64;
+std::mutex g_split_mu;
+SplitRegion g_split_region[kSplitDevices][kSplitRegions];
+void* g_split_base[kSplitDevices] = {};
+int g_split_next[kSplitDevices] = {};
+
+// Under g_split_mu: a region of the current device the stream may write next,
+// or nullptr.
+float* split_take(int dev, hipStream_t st, SplitRegion** out) {
+  if (g_split_base[dev] == nullptr) {
+    void* p = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(split_scratch)) != hipSuccess) return nullptr;
+    for (SplitRegion& r : g_split_region[dev])
+      if (r.done == nullptr &&
+          hipEventCreateWithFlags(&r.done, hipEventDisableTiming) != hipSuccess)
+        return nullptr;
+    g_split_base[dev] = p;
+  }
+  int pick = -1;
+  for (int i = 0; i < kSplitRegions && pick < 0; ++i) {
+    const SplitRegion& r = g_split_region[dev][i];
+    if (!r.used || r.last == st) pick = i;
+  }
+  for (int i = 0; i < kSplitRegions && pick < 0; ++i)
+    if (hipEventQuery(g_split_region[dev][i].done) == hipSuccess) pick = i;
+  if (pick < 0) {
+    pick = g_split_next[dev];
+    g_split_next[dev] = (pick + 1) % kSplitRegions;
+  }
+  (void)hipGetLastError();  // (an event that has not ended is reported as an error)
+  SplitRegion& r = g_split_region[dev][pick];
+  if (r.used && hipStreamWaitEvent(st, r.done, 0) != hipSuccess) return nullptr;
+  *out = &r;
+  return (float*)((char*)g_split_base[dev] + (size_t)pick * kSplitRegionBytes);
+}
+
+// The split kernels where they pay: caches of more than 768 rows, several
+// query heads per kv head.  Not while the stream is captured (a replay would
+// use the region without taking it) and not without a region: -1, the caller
+// launches the one-launch kernel, which takes every shape.
+constexpr int kSplitMinRows = 768;
+
+int gqa_split(const void* qkv, const float* qkv_parts, int n_parts, const void* q_norm,
+              const void* k_norm, const float* cos_t, const float* sin_t, const int64_t* pos, int c,
+              int nh, int kvh, int L, float eps, float scale, void* k_cache, void* v_cache,
+              void* out, hipStream_t st) {
+  const int grp = nh / kvh, zh = (grp + kSplitHeads - 1) / kSplitHeads;
+  if (L <= kSplitMinRows || grp < 2 || kvh > 65535 || nh > 65535) return -1;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  int dev = 0;
+  if (hipStreamIsCapturing(st, &cap) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
+    (void)hipGetLastError();
+    return -1;
+  }
+  if (cap != hipStreamCaptureStatusNone || dev < 0 || dev >= kSplitDevices) return -1;
+  // three workgroups per CU, at least 128 rows each
+  const long units = (long)c * kvh * zh;
+  const int splits = (int)std::max(1L, std::min({768 / units, (long)kSplitMax, (long)L / 128}));
+  if ((size_t)c * nh * splits * kSplitRec * sizeof(float) > kSplitRegionBytes) return -1;
+  std::lock_guard<std::mutex> lock(g_split_mu);
+  SplitRegion* region = nullptr;
+  float* part = split_take(dev, st, &region);
+  if (part == nullptr) {
+    (void)hipGetLastError();
+    return -1;
+  }
+  hipLaunchKernelGGL(gqa_split_kernel, dim3(c * zh, kvh, splits), dim3(kSplitWaves * 64), 0, st,
+                     (const uint16_t*)qkv, qkv_parts, n_parts, (const uint16_t*)q_norm,
+                     (const uint16_t*)k_norm, cos_t, sin_t, pos, nh, kvh, zh, L, eps, scale,
+                     (uint16_t*)k_cache, (uint16_t*)v_cache, part);
+  hipLaunchKernelGGL(gqa_merge_kernel, dim3(c, nh), dim3(kT), 0, st, (const float*)part, pos, nh,
+                     splits, L, (uint16_t*)out);
+  const hipError_t launched = hipGetLastError(), marked = hipEventRecord(region->done, st);
+  region->used = true;
+  region->last = st;
+  return (int)(launched != hipSuccess ? launched : marked);
+}
+
+}  // namespace
+
 extern "C" int sluice_dec_gqa_decode(const void* qkv, const float* qkv_parts, int n_parts,
                                      const void* q_norm, const void* k_norm,
                                      const float* cos_t, const float* sin_t, const int64_t* pos,
@@ -1507,6 +1897,9 @@ extern "C" int sluice_dec_gqa_decode(const void* qkv, const float* qkv_parts, in
       ((uintptr_t)out & 3) != 0)
     return SLUICE_E_INVAL;
   if (c == 0) return SLUICE_OK;
+  const int split = gqa_split(qkv, qkv_parts, n_parts, q_norm, k_norm, cos_t, sin_t, pos, c, nh,
+                              kvh, L, eps, scale, k_cache, v_cache, out, (hipStream_t)stream);
+  if (split >= 0) return split;
   hipLaunchKernelGGL((gqa_decode_kernel<kGqaWaves, kGqaRows>), dim3(c, nh),
                      dim3(kGqaWaves * 64), 0, (hipStream_t)stream, (const uint16_t*)qkv,
                      qkv_parts, n_parts, (const uint16_t*)q_norm, (const uint16_t*)k_norm, cos_t, sin_t, pos, nh, kvh,

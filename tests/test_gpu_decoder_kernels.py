@@ -428,3 +428,95 @@ def test_gqa_decode(L, positions):
     for name, ref in (("k", k), ("v", v)):
         got = d[name].cpu().permute(0, 2, 1, 3)
         assert torch.equal(got[mask], ref.permute(0, 2, 1, 3)[mask]), name
+
+
+@pytest.mark.parametrize("nh,kvh,L,parts", [(32, 4, 800, 0), (8, 4, 4096, 0), (16, 1, 1056, 3),
+                                            (40, 2, 769, 0), (32, 16, 2080, 0)])
+def test_gqa_decode_split_matches_the_one_launch_kernel(nh, kvh, L, parts):
+    """Long caches run split over the rows in two launches; while a stream is
+    captured the one-launch kernel runs.  Both keep the softmax in fp32, so the
+    bf16 outputs are at most one rounding apart (2^-8); the cache rows have the
+    same bits.  Rows past a position hold NaN: they have no weight.  Positions
+    outside the cache write nothing."""
+    lib, check = _lib()
+    hd = 128
+    positions = [0, 1, 31, 32, 127, 128, 129, 511, L - 1, -1, L]
+    c = len(positions)
+    g = torch.Generator(device=DEV).manual_seed(nh + L)
+
+    def rand(shape):
+        return torch.randn(shape, generator=g, device=DEV).bfloat16()
+
+    qkv = rand((c, (nh + 2 * kvh) * hd))
+    pt = torch.stack([qkv.float() / 4, qkv.float() / 4, qkv.float() / 2]) if parts else None
+    qn, kn = 1 + 0.1 * rand((hd,)), 1 + 0.1 * rand((hd,))
+    k, v = rand((c, kvh, L, hd)), rand((c, kvh, L, hd))
+    for t, p in enumerate(positions):
+        k[t, :, max(p, 0):], v[t, :, max(p, 0):] = float("nan"), float("nan")
+    pos = torch.tensor(positions, dtype=torch.long, device=DEV)
+    cos_t, sin_t = (a.to(DEV) for a in _tables(L, hd, 1e6))
+
+    def call(k, v, out):
+        check(lib.sluice_dec_gqa_decode(
+            None if parts else qkv.data_ptr(), pt.data_ptr() if parts else None, parts,
+            qn.data_ptr(), kn.data_ptr(), cos_t.data_ptr(), sin_t.data_ptr(), pos.data_ptr(), c, nh,
+            kvh, hd, L, 1e-6, hd ** -0.5, k.data_ptr(), v.data_ptr(), out.data_ptr(), _st()),
+            "gqa_decode")
+
+    k1, v1 = k.clone(), v.clone()
+    outs = []
+    for _ in range(2):  # the second call reuses the first one's scratch
+        outs.append(torch.full((c, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV))
+        call(k1, v1, outs[-1])
+    k2, v2 = k.clone(), v.clone()
+    ref = torch.full_like(outs[0], 7.0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(k2, v2, ref)
+    # the one-launch kernel weighs rows past the position with 0, NaN or not
+    k2[torch.isnan(k2)], v2[torch.isnan(v2)] = 0, 0
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
+    for t, p in enumerate(positions):
+        if not 0 <= p < L:
+            assert (outs[0][t] == 7.0).all() and (ref[t] == 7.0).all()
+            continue
+        assert _rel(outs[0][t], ref[t].float().cpu()) <= 2.0 ** -8, (t, p)
+        assert torch.equal(k1[t, :, p], k2[t, :, p]) and torch.equal(v1[t, :, p], v2[t, :, p])
+        assert torch.isnan(k1[t, :, p + 1:]).all() and torch.equal(k1[t, :, :p], k[t, :, :p])
+
+
+def test_gqa_decode_split_on_more_streams_than_scratch_regions():
+    """Calls in flight on more streams than there are scratch regions give the
+    bits they give one after another."""
+    lib, check = _lib()
+    nh, kvh, L, c, hd, n = 32, 4, 2048, 4, 128, 6
+    g = torch.Generator(device=DEV).manual_seed(5)
+    cos_t, sin_t = (a.to(DEV) for a in _tables(L, hd, 1e6))
+    w = torch.ones(hd, dtype=torch.bfloat16, device=DEV)
+    pos = torch.tensor([2047, 1500, 900, 10], device=DEV)
+    qkv = [torch.randn((c, (nh + 2 * kvh) * hd), generator=g, device=DEV).bfloat16()
+           for _ in range(n)]
+    k, v = ([torch.randn((c, kvh, L, hd), generator=g, device=DEV).bfloat16() for _ in range(n)]
+            for _ in range(2))
+    out = torch.zeros((2, n, c, nh * hd), dtype=torch.bfloat16, device=DEV)
+
+    def call(i, o):
+        check(lib.sluice_dec_gqa_decode(
+            qkv[i].data_ptr(), None, 0, w.data_ptr(), w.data_ptr(), cos_t.data_ptr(),
+            sin_t.data_ptr(), pos.data_ptr(), c, nh, kvh, hd, L, 1e-6, hd ** -0.5, k[i].data_ptr(),
+            v[i].data_ptr(), o.data_ptr(), _st()), "gqa_decode")
+
+    for i in range(n):
+        call(i, out[0, i])
+        torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(device=DEV) for _ in range(n)]
+    for _ in range(20):
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                call(i, out[1, i])
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], out[1])
