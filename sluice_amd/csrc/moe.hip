@@ -174,16 +174,11 @@ struct ItemLds {
 // multiplied by its scale before it joins the accumulator.
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ uint32_t pack_bf16_hi(float a, float b) {
-  // fp8 values are exact in bf16: keep the top 16 bits of each fp32.
-  return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & 0xffff0000u);
-}
-
-// 4 fp8 bytes -> 4 bf16 (two dwords).
+// 4 fp8 bytes -> 4 bf16 (two dwords); every fp8 value is exact in bf16.
 __device__ __forceinline__ u32x2_t fp8x4_to_bf16x4(uint32_t v) {
-  const f32x2_t lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(v, 1.0f, false);
-  const f32x2_t hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(v, 1.0f, true);
-  return u32x2_t{pack_bf16_hi(lo.x, lo.y), pack_bf16_hi(hi.x, hi.y)};
+  return u32x2_t{
+      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, false)),
+      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(v, 1.0f, true))};
 }
 
 __device__ __forceinline__ void fp8x16_to_bf16(u32x4_t q, u32x4_t& lo, u32x4_t& hi) {
@@ -686,7 +681,7 @@ __host__ __device__ inline int g2_groups(int H, bool fp8) {
 }
 
 template <bool FP8>
-__global__ __launch_bounds__(kThreads) void moe_gemm2_kernel(const uint16_t* __restrict__ act,
+__global__ __launch_bounds__(kThreads, 4) void moe_gemm2_kernel(const uint16_t* __restrict__ act,
                                                              ExpertW W,
                                                              const int32_t* __restrict__ plan,
                                                              const float* __restrict__ topk_w,
@@ -739,8 +734,11 @@ __device__ __forceinline__ void wait_count(const int32_t* count, int want, const
 // host's ready marks, so the waits end whatever order the hardware
 // dispatches workgroups in.  The grid must cover every item (the host sizes
 // it for the largest plan of the call); workgroups beyond the items exit.
+// (120 VGPRs: at its 4 waves per SIMD the copy kernel's room stays free, see
+// build.py.)
 template <bool FP8>
-__global__ __launch_bounds__(kThreads) void moe_gemm2_split_kernel(
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_num_vgpr(120))) void moe_gemm2_split_kernel(
     const uint16_t* __restrict__ x, uint16_t* __restrict__ act, ExpertW W,
     const int32_t* __restrict__ plan, const float* __restrict__ topk_w, CallShape cs,
     float* __restrict__ partial, int32_t* __restrict__ handoff) {

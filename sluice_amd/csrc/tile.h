@@ -22,7 +22,8 @@
 // with the LDS reads scheduled between the products).  Whole calls against the
 // decode kernels: Qwen3 shape, 4096 tokens, 4084 -> 570 us; V2-Lite
 // shape, 509 tokens over 48 slots, 628 -> 229 us; V3 fp8, 384 tokens over 64 of
-// 256 experts, 1364 -> 725 us.
+// 256 experts, 1493 -> 717 us (rows past a tile's pairs not loaded, and fp8
+// widened to bf16 by one instruction per pair: 725 -> 698 side by side).
 //
 // LDS rows are 128 bytes (64 bf16 or 128 fp8 of K) in eight 16-byte
 // segments, segment s of row r at s ^ (r & 7); the swizzle is in the lanes'
@@ -224,6 +225,8 @@ struct TileCfg {
   static constexpr int kStage = CH * 128 + BM * KS * 2;
   static constexpr int NA = CH / 8 / NW, NB = BM / 8 * SUB / NW;  // DMAs per wave and stage
   static constexpr int kOut = G1 ? CH / 2 : CH;   // output channels per item
+  // DMAs of a stage that load the rows of ng fragments per wave column.
+  static constexpr int loads(int ng) { return (2 * ng * WP * SUB + NW - 1) / NW; }
   static_assert(NA * NW * 8 == CH && NB * NW * 8 == BM * SUB && FM % 2 == 0, "tile split");
 };
 
@@ -273,13 +276,23 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
     const TileRec rec = ldu(a.plan.tiles + ft + (local - cb * nt));
     return Item{rec.slot_field, rec.pos0, rec.count, cb};
   };
+  // This wave's i-th token DMA of a stage: 8 rows of sub-tile token_sub(i),
+  // lower rows first, so that a tile with few pairs loads few rows.
+  auto token_sub = [&](int i) { return (wave + i * NW) % C::SUB; };
+  auto token_group = [&](int i) { return (wave + i * NW) / C::SUB; };
+  // The fragments per wave column that hold an item's pairs, rounded up to
+  // the K loops there are.
+  auto fragments = [&](int count) {
+    const int n = (((count + 15) >> 4) + C::WP - 1) / C::WP;
+    constexpr int kUnit = FN >= 4 ? FN / 4 : FN / 2;
+    return (n + kUnit - 1) / kUnit * kUnit;
+  };
   // The rows this lane loads of an item: pairs (gemm1; turned into tokens when
   // they are used, so that nothing waits for them here) or sorted positions.
   auto rows_of = [&](const Item& it, int (&rows)[C::NB]) {
 #pragma unroll
     for (int i = 0; i < C::NB; ++i) {
-      const int g = (wave + i * NW) % (BM / 8);
-      const int row = min(g * 8 + (lane >> 3), it.count - 1);
+      const int row = min(token_group(i) * 8 + (lane >> 3), it.count - 1);
       rows[i] = G1 ? (int)a.plan.order[it.pos0 + row] : row;
     }
   };
@@ -341,13 +354,12 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < C::NB; ++i) {
-      const int sub = (wave + i * NW) / (BM / 8);
       uint32_t row = (uint32_t)rows[i];
       if (G1)  // pair / k is exact: pairs are below 2^16
         row = slot >= a.W.S      ? row - (uint32_t)(a.cs.T * a.cs.k + (slot - a.W.S) * a.cs.T)
               : a.cs.k > 1 ? __umulhi(row, by_k)
                            : row;
-      vb[i] = row * (uint32_t)(K * 2) + (uint32_t)(sub * 128 + bseg * 16);
+      vb[i] = row * (uint32_t)(K * 2) + (uint32_t)(token_sub(i) * 128 + bseg * 16);
     }
     k0 = first_chunk(it);
   };
@@ -356,20 +368,23 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
   // workgroups that all read the same columns meet in the same memory
   // channels.  (k0 depends on the weights alone, so a pair's sum has one
   // order whichever tile it lands in.)
-  auto issue = [&](int k, int buf) {
+  auto issue = [&](int k, int buf, int nb) {
     const int kk = k + k0 < nk ? k + k0 : k + k0 - nk;
     const uint8_t* ap = abase + (size_t)kk * 128;
     const uint8_t* bp = bbase + (size_t)kk * (C::KS * 2);
-    const uint32_t d = lds0 + (uint32_t)(buf * C::kStage) + (uint32_t)wave * 1024;
+    const uint32_t d = lds0 + (uint32_t)(buf * C::kStage);
 #pragma unroll
-    for (int i = 0; i < C::NA; ++i) dma16(d + i * NW * 1024, ap, va[i]);
+    for (int i = 0; i < C::NA; ++i) dma16(d + (wave + i * NW) * 1024, ap, va[i]);
 #pragma unroll
-    for (int i = 0; i < C::NB; ++i) dma16(d + CH * 128 + i * NW * 1024, bp, vb[i]);
+    for (int i = 0; i < C::NB; ++i)
+      if (i < nb)
+        dma16(d + CH * 128 + token_sub(i) * (BM * 128) + token_group(i) * 1024, bp, vb[i]);
   };
-  auto issue_first = [&]() {
+  auto issue_first = [&](int count) {
+    const int nb = C::loads(fragments(count));
 #pragma unroll
     for (int s = 0; s < ST - 1; ++s)
-      if (s < nk) issue(s, s);
+      if (s < nk) issue(s, s, nb);
   };
 
   int n = rank;
@@ -381,7 +396,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
   if (FP8) nsc = scales_of(it, first_chunk(it) >> 6);
   await_slot(a.W.wait, it.slot_field);
   address(it, rows);
-  issue_first();
+  issue_first(it.count);
   for (;;) {
     const int next = n + per_xcd;
     const bool more = next < rn + sn;
@@ -410,7 +425,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
       constexpr int NG = decltype(ng)::value;
       int buf = 0;
       for (int k = 0; k < nk; ++k) {
-        constexpr int L = C::NA + C::NB;
+        constexpr int nb = C::loads(NG), L = C::NA + nb;
         const int ahead = min(ST - 2, nk - 1 - k);  // stages after k in flight
         if (ST >= 4 && ahead >= 2)
           dma_wait<(ST >= 4 ? 2 * L : 0)>();
@@ -418,7 +433,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
           dma_wait<(ST >= 3 ? L : 0)>();
         else
           dma_wait<0>();
-        if (k + ST - 1 < nk) issue(k + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+        if (k + ST - 1 < nk) issue(k + ST - 1, buf == 0 ? ST - 1 : buf - 1, nb);
         const uint8_t* sa = lds + buf * C::kStage + (wc * C::CW + R) * 128;
         const uint8_t* sb = lds + buf * C::kStage + CH * 128 + (wp * 16 + R) * 128;
         auto ldl = [](const uint8_t* p) { return *reinterpret_cast<const u32x4_t*>(p); };
@@ -479,12 +494,12 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
         buf = buf + 1 == ST ? 0 : buf + 1;
       }
     };
-    const int groups = (((count + 15) >> 4) - wp + C::WP - 1) / C::WP;  // of this wave
-    if (FN >= 4 && groups <= FN / 4)
+    const int ng = fragments(count);
+    if (FN >= 4 && ng == FN / 4)
       k_loop(std::integral_constant<int, (FN >= 4 ? FN / 4 : FN)>{});
-    else if (groups <= FN / 2)
+    else if (ng == FN / 2)
       k_loop(std::integral_constant<int, FN / 2>{});
-    else if (FN >= 4 && groups <= FN * 3 / 4)
+    else if (FN >= 4 && ng == FN * 3 / 4)
       k_loop(std::integral_constant<int, (FN >= 4 ? FN * 3 / 4 : FN)>{});
     else
       k_loop(std::integral_constant<int, FN>{});
@@ -492,7 +507,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
       dma_wait<0>();  // every wave has read its last stage
       await_slot(a.W.wait, nit.slot_field);
       address(nit, rows);
-      issue_first();
+      issue_first(nit.count);
     }
     // Epilogue: column R of fragment g is pair pos0 + 16 (g WP + wp) + R, rows
     // 4 kb .. +4 of fragment f its channels.
