@@ -31,7 +31,10 @@ _MAX_PREFILL_WORKSPACE = 1 << 30  # bytes; larger chunks run in slices
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle (without the Stream object that
+    torch.cuda.current_stream makes: 0.1 against 1.9 us)."""
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -298,9 +301,39 @@ def _(hidden_states, w1, w2, topk_weights, topk_ids, activation="silu", global_n
     return torch.empty_like(hidden_states)
 
 
+def _nothing_watches(tensors) -> bool:
+    """No transform, mode, tracer, profiler or gradient would see an op called
+    on these arguments: the op then does nothing but call its body."""
+    if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._get_tracing_state() is not None
+            or torch.autograd._profiler_enabled()
+            or torch.autograd.forward_ad._current_level >= 0):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is None:
+            continue
+        if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
+            return False
+        if t.device.type != "cuda" or (grad and t.requires_grad):
+            return False
+    return True
+
+
 def fused_experts(hidden_states, w1, w2, topk_weights, topk_ids, activation="silu",
                   global_num_experts=-1, expert_map=None, **kw):
-    """Keyword surface of vLLM's fused_experts as the router-split entry uses it."""
+    """Keyword surface of vLLM's fused_experts as the router-split entry uses it.
+
+    An eager call that nothing watches goes to the op's body directly: the
+    dispatch through the Python op costs 8 of its 25 us."""
+    if _nothing_watches((hidden_states, w1, w2, topk_weights, topk_ids, expert_map)) and (
+            not kw or _nothing_watches([v for v in kw.values() if isinstance(v, torch.Tensor)])):
+        return _fused_experts_impl(
+            hidden_states, w1, w2, topk_weights, topk_ids, activation, global_num_experts,
+            expert_map, kw.pop("w1_scale", None), kw.pop("w2_scale", None),
+            kw.pop("block_shape", None), kw.pop("routed_scaling_factor", 1.0),
+            kw.pop("shared_output", None), **kw)
     return torch.ops.sluice.fused_experts(hidden_states, w1, w2, topk_weights, topk_ids,
                                           activation=activation,
                                           global_num_experts=global_num_experts,

@@ -531,3 +531,36 @@ def test_tiled_product_over_a_map_whose_slots_streamed():
         assert om.rel_l2(got.float().cpu().numpy(), ref.float().cpu().numpy()) <= ONE_ROUNDING
     finally:
         off.close()
+
+
+def test_fused_experts_goes_through_the_op_when_something_watches():
+    """A dispatch mode, the profiler and autograd see the op; a plain eager
+    call gives its bits without it; make_fx and vmap-free tracing get one node."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from sluice_amd import ops
+
+    args, kw = _tile_case(3, 256, 64, 64, 8, 8, 2, 1.0, False, seed=8)
+    want = torch.ops.sluice.fused_experts(*args, **kw)
+    assert torch.equal(ops.fused_experts(*args, **kw), want)
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, a=(), k=None):
+            seen.append(str(func))
+            return func(*a, **(k or {}))
+
+    with Watch():
+        assert torch.equal(ops.fused_experts(*args, **kw), want)
+    assert any("fused_experts" in s for s in seen)
+    g = make_fx(lambda x: ops.fused_experts(x, *args[1:], **kw))(args[0])
+    assert any("fused_experts" in str(n.target) for n in g.graph.nodes)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        ops.fused_experts(*args, **kw)
+    assert any("fused_experts" in e.key for e in prof.key_averages())
+    x = args[0].clone().requires_grad_()
+    assert ops.fused_experts(x, *args[1:], **kw).requires_grad == torch.ops.sluice.fused_experts(
+        x, *args[1:], **kw).requires_grad
+    with pytest.raises(TypeError):
+        ops.fused_experts(*args, **kw, no_such_argument=1)
