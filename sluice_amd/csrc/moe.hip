@@ -674,6 +674,130 @@ __global__ __launch_bounds__(kThreads) void moe_gemm1_kernel(const uint16_t* __r
   }
 }
 
+// gemm1 of a small call that has no plan yet (P <= kSelfPairs pairs, no slot
+// of the map may stream): every workgroup groups the pairs by itself -- one pair
+// per thread, every 16th pair of a slot leads a block -- and one more workgroup, the last, writes the plan that gemm2 and
+// the combine read.  The align launch goes (4.9 us and a launch gap) for two
+// dependent loads (ids, map) and five barriers at the head of each workgroup.
+// Replayed calls, with the align launch and without: V2-Lite 39.3 / 36.6 us
+// for one token, 78.9 / 77.8 for 8, 91.5 / 92.6 for 12; Qwen3 30.0 / 26.9 for
+// one, 66.1 / 64.1 for 12 (96 pairs, the line), 73.2 / 72.9 for 16; V3 fp8 217
+// / 214 for 8.  (Counting each pair's rank against all the others' slots
+// instead of by LDS atomics: 77 us for 12 tokens.)  The shared blocks come
+// first, since their number is known.
+constexpr int kSelfPairs = 96;
+static_assert(kSelfPairs <= kThreads, "a pair per thread");
+
+struct SelfPlan {
+  int slots[kSelfPairs];           // of the pairs, -1 = not resident
+  int cnt[SLUICE_MAX_SLOTS];       // a slot's pairs
+  int lead[SLUICE_MAX_SLOTS];      // its first pair
+  int first[SLUICE_MAX_SLOTS];     // the block of its first 16 pairs
+  int wsum[kKS];
+  int slot, rb, pair[kBM];
+};
+
+template <bool FP8>
+__global__ __launch_bounds__(kThreads) void moe_gemm1_self_kernel(
+    const uint16_t* __restrict__ x, ExpertW W, const int32_t* __restrict__ ids,
+    const int32_t* __restrict__ map, int E, CallShape cs, uint16_t* __restrict__ act,
+    int32_t* __restrict__ plan) {
+  __shared__ ItemLds lds;
+  __shared__ SelfPlan sp;
+  const int tid = threadIdx.x, wave = tid >> 6, P = cs.T * cs.k;
+  int slot = -1;
+  if (tid < P) {
+    const int g = ids[tid];
+    if ((unsigned)g < (unsigned)E) slot = map != nullptr ? map[g] : g;
+    if ((unsigned)slot >= (unsigned)W.S) slot = -1;
+  }
+  if (slot >= 0) {
+    sp.cnt[slot] = 0;
+    sp.lead[slot] = kThreads;
+  }
+  if (tid < kSelfPairs) sp.slots[tid] = slot;
+  __syncthreads();
+  // Every workgroup must come to the same blocks: a slot's first pair leads
+  // its block, whose columns may be in any order (the LDS atomics')...
+  int rank = 0;
+  if (slot >= 0) {
+    rank = atomicAdd(&sp.cnt[slot], 1);
+    atomicMin(&sp.lead[slot], tid);
+  }
+  const int over = __syncthreads_or(rank >= kBM);
+  const int count = slot >= 0 ? sp.cnt[slot] : 0;
+  bool leads = slot >= 0 && sp.lead[slot] == tid;
+  if (over) {
+    // ...unless a slot has several, which then take its pairs in pair order.
+    rank = 0;
+    for (int j = 0; j < tid && slot >= 0; ++j) rank += sp.slots[j] == slot ? 1 : 0;
+    leads = slot >= 0 && (rank & (kBM - 1)) == 0;
+  }
+  const uint64_t m = __ballot(leads);
+  if ((tid & 63) == 0) sp.wsum[wave] = __popcll(m);
+  __syncthreads();
+  int block = mask_rank(m), nr = 0;  // of a leader; the routed blocks
+#pragma unroll
+  for (int w = 0; w < kKS; ++w) {
+    if (w < wave) block += sp.wsum[w];
+    nr += sp.wsum[w];
+  }
+  if (blockIdx.x == gridDim.x - 1) {
+    int32_t* blocks = plan + kPlanHeader;
+    if (slot >= 0 && sp.lead[slot] == tid) sp.first[slot] = block;
+    __syncthreads();
+    if (tid < P) blocks[(size_t)kBlockInts * P + tid] = slot >= 0 ? 1 : 0;
+    if (leads) {
+      blocks[(size_t)block * kBlockInts] = slot;
+      blocks[(size_t)block * kBlockInts + 1] = over ? min(kBM, count - rank) : count;
+    }
+    // a slot's further blocks (more than 16 pairs of it) are told one by one
+    for (int b = 0; over && b < nr; ++b) {
+      if (leads && block == b) {
+        sp.slot = slot;
+        sp.rb = rank / kBM;
+      }
+      __syncthreads();
+      const bool mine = slot >= 0 && rank >= kBM && slot == sp.slot && rank / kBM == sp.rb;
+      if (mine) blocks[(size_t)b * kBlockInts + 2 + rank % kBM] = tid;
+      __syncthreads();
+    }
+    if (slot >= 0 && rank < kBM)
+      blocks[(size_t)sp.first[slot] * kBlockInts + 2 + rank] = tid;
+    if (tid == 0) {
+      plan[0] = nr;
+      plan[1] = P;
+      plan[2] = nr;
+      plan[3] = 0;
+    }
+    return;
+  }
+  const int n_tiles = cs.I / 16, per = (cs.T + kBM - 1) / kBM, n_shb = W.I_s / cs.I * per;
+  const int total = (n_shb + nr) * n_tiles, col = tid & 15;
+  for (int item = blockIdx.x; item < total; item += gridDim.x - 1) {
+    const int b = item / n_tiles, tile = item - b * n_tiles;
+    int s, pair;
+    if (b < n_shb) {
+      const int v = b / per, t = (b - v * per) * kBM + col;
+      s = W.S + v;
+      pair = t < cs.T ? P + v * cs.T + t : -1;
+    } else {
+      if (leads && block == b - n_shb) {
+        sp.slot = slot;
+        sp.rb = over ? rank / kBM : 0;
+      }
+      if (tid < kBM) sp.pair[tid] = -1;
+      __syncthreads();
+      s = sp.slot;
+      if (slot == s && rank / kBM == sp.rb) sp.pair[rank % kBM] = tid;
+      __syncthreads();
+      pair = sp.pair[col];
+    }
+    s = __builtin_amdgcn_readfirstlane(s);
+    run_g1<FP8>(x, W, cs, s, pair, tile, act, lds);
+  }
+}
+
 __host__ __device__ inline int g2_groups(int H, bool fp8) {
   const int n_tiles = H / (16 * kG2T);
   const int R = fp8 ? G2Shape<true>::R : G2Shape<false>::R;
@@ -1102,7 +1226,10 @@ int run_experts(const void* x, const ExpertW& W, const float* tw, const int32_t*
   const int bm = plan == nullptr ? tile_pairs<FP8>(cs, E, S) : 0;
   if (bm > 0)
     return run_tiled<FP8>(x, Ww, tw, ti, map, cs, E, S, n_sh, bm, scale, shared, w, out, st);
-  if (plan == nullptr) {
+  const bool self = plan == nullptr && Ww.wait.pending == nullptr && P <= kSelfPairs;
+  if (self) {
+    plan = w.plan;
+  } else if (plan == nullptr) {
     hipLaunchKernelGGL(moe_align_kernel, dim3(1), dim3(kThreads), 0, st, ti, P, map, E, S,
                        Ww.wait.pending, w.plan);
     SLUICE_HIP_CHECK(hipGetLastError());
@@ -1133,8 +1260,12 @@ int run_experts(const void* x, const ExpertW& W, const float* tw, const int32_t*
       g1 = std::min(g1, c1);
       g2 = std::min(g2, c2);
     }
-    hipLaunchKernelGGL((moe_gemm1_kernel<FP8>), dim3(g1), dim3(kThreads), 0, st,
-                       (const uint16_t*)x, Ww, plan, cs, w.act, (int32_t*)nullptr);
+    if (self)
+      hipLaunchKernelGGL((moe_gemm1_self_kernel<FP8>), dim3(g1 + 1), dim3(kThreads), 0, st,
+                         (const uint16_t*)x, Ww, ti, map, E, cs, w.act, w.plan);
+    else
+      hipLaunchKernelGGL((moe_gemm1_kernel<FP8>), dim3(g1), dim3(kThreads), 0, st,
+                         (const uint16_t*)x, Ww, plan, cs, w.act, (int32_t*)nullptr);
     SLUICE_HIP_CHECK(hipGetLastError());
     hipLaunchKernelGGL((moe_gemm2_kernel<FP8>), dim3(g2), dim3(kThreads), 0, st, w.act, Ww, plan,
                        tw, cs, w.partial);

@@ -564,3 +564,40 @@ def test_fused_experts_goes_through_the_op_when_something_watches():
         x, *args[1:], **kw).requires_grad
     with pytest.raises(TypeError):
         ops.fused_experts(*args, **kw, no_such_argument=1)
+
+
+@pytest.mark.parametrize("T,k,E,S,how", [
+    (1, 1, 1, 1, "even"),          # one pair
+    (1, 6, 64, 48, "even"),
+    (12, 8, 128, 96, "even"),      # 96 pairs: the largest call that plans itself
+    (97, 1, 64, 64, "even"),       # 97 pairs: the align launch
+    (31, 3, 4, 4, "even"),         # about 23 pairs per slot: a block and a rest
+    (48, 2, 16, 16, "one"),        # every pair to one expert: six full blocks
+    (9, 8, 512, 512, "even"),
+    (9, 4, 16, 8, "outside"),      # no pair is resident
+])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_small_calls_plan_themselves(T, k, E, S, how, fp8):
+    """Without a plan a small call groups its pairs in gemm1; the bits are
+    those of the stages run over an align plan."""
+    from sluice_amd import _lib, ops
+
+    H, I = 256, 128
+    args, kw = _tile_case(T, H, I, 0, E, S, k, 0.9 if S < E else 1.0, fp8, seed=T + E) \
+        if T > 1 else _tile_case(2, H, I, 0, E, S, k, 1.0, fp8, seed=E)
+    x, w13, w2, tw, ids = args
+    x, tw, ids = x[:T].contiguous(), tw[:T].contiguous(), ids[:T].contiguous()
+    if how == "one":
+        ids[:] = 3
+    elif how == "outside":
+        ids[:] = -1
+    kw["routed_scaling_factor"] = 1.0
+    st = torch.cuda.current_stream().cuda_stream
+    ref = _staged(_lib.load(), x, w13, w2, tw, ids, kw["expert_map"], T, H, I, E, S, k, 1.0, None,
+                  st, fp8=(kw["w1_scale"], kw["w2_scale"]) if fp8 else None)
+    for _ in range(3):
+        got = ops.fused_experts(x, w13, w2, tw, ids, **kw)
+        torch.cuda.synchronize()
+        assert torch.equal(got, ref)
+    if how != "outside":
+        assert (ref != 0).any()
