@@ -689,9 +689,14 @@ __global__ __launch_bounds__(kMlaWaves * 64) void mla_partial_kernel(
 // of out = o_lat . w_uv[h]: a thread owns 8 columns and 16 latent rows (lane
 // group and wave pick the rows), the 32 row groups meet in LDS.  Everything
 // whose address does not depend on the position goes out first: the w_uv
-// rows, every split's (max, sum) and the first 8 splits' partial sums (splits
-// past the position are never used, so whatever they hold is harmless:
-// they are selected away, not multiplied by 0).
+// rows, every split's (max, sum) and the first kMlaPre splits' partial sums
+// (splits past the position are never used, so whatever they hold is
+// harmless: they are selected away, not multiplied by 0).  Each further pass
+// over the splits is a memory round trip: 16 at a time against 8 took the
+// three launches from 19.2 to 18.2 us for 8 tokens of 120 to 1023 rows, from
+// 28.2 to 27.2 for 1000 to 4095 (and from 12.4 to 12.5 for one token of 128 to
+// 383).
+constexpr int kMlaPre = 16;
 __global__ __launch_bounds__(kT) void mla_merge_kernel(const float* __restrict__ part,
                                                        const uint16_t* __restrict__ w_uv,
                                                        const int64_t* __restrict__ pos, int nh,
@@ -710,9 +715,9 @@ __global__ __launch_bounds__(kT) void mla_merge_kernel(const float* __restrict__
   const float* rec = part + ((size_t)t * kMlaSplit * nh + h) * kMlaRec;
   const size_t sstride = (size_t)nh * kMlaRec;
   static_assert(2 * kT == kLora, "two latent columns per thread");
-  f32x2_t pv[8];  // splits 0..7, columns 2 * tid, 2 * tid + 1
+  f32x2_t pv[kMlaPre];  // the first splits, columns 2 * tid, 2 * tid + 1
 #pragma unroll
-  for (int u = 0; u < 8; ++u)
+  for (int u = 0; u < kMlaPre; ++u)
     pv[u] = *reinterpret_cast<const f32x2_t*>(rec + u * sstride + 4 + 2 * tid);
   float ms = -INFINITY, ls = 0.f;
   if (tid < kMlaSplit) {
@@ -735,20 +740,20 @@ __global__ __launch_bounds__(kT) void mla_merge_kernel(const float* __restrict__
   {
     float v0 = 0.f, v1 = 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < kMlaPre; ++u) {
       if (u < na) {
         v0 += ws[u] * pv[u][0];
         v1 += ws[u] * pv[u][1];
       }
     }
-    for (int s0 = 8; s0 < na; s0 += 8) {
+    for (int s0 = kMlaPre; s0 < na; s0 += kMlaPre) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < kMlaPre; ++u) {
         const int sp = s0 + u < na ? s0 + u : 0;
         pv[u] = *reinterpret_cast<const f32x2_t*>(rec + sp * sstride + 4 + 2 * tid);
       }
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
+      for (int u = 0; u < kMlaPre; ++u) {
         if (s0 + u < na) {
           v0 += ws[s0 + u] * pv[u][0];
           v1 += ws[s0 + u] * pv[u][1];
