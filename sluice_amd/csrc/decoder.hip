@@ -1799,7 +1799,8 @@ namespace {
 // event marks their end and the next call's stream waits for it, so calls on
 // any streams and threads are kept apart (a wait on the call's own stream
 // costs nothing on the device).  A call prefers the region its stream used
-// last, then one whose last call has ended.
+// last, then one not used yet, then takes them in turn.  (No event is queried:
+// a query is not allowed while another thread captures a graph.)
 struct SplitRegion {
   hipEvent_t done = nullptr;
   hipStream_t last = nullptr;
@@ -1826,15 +1827,14 @@ float* split_take(int dev, hipStream_t st, SplitRegion** out) {
   int pick = -1;
   for (int i = 0; i < kSplitRegions && pick < 0; ++i) {
     const SplitRegion& r = g_split_region[dev][i];
-    if (!r.used || r.last == st) pick = i;
+    if (r.used && r.last == st) pick = i;
   }
   for (int i = 0; i < kSplitRegions && pick < 0; ++i)
-    if (hipEventQuery(g_split_region[dev][i].done) == hipSuccess) pick = i;
+    if (!g_split_region[dev][i].used) pick = i;
   if (pick < 0) {
     pick = g_split_next[dev];
     g_split_next[dev] = (pick + 1) % kSplitRegions;
   }
-  (void)hipGetLastError();  // (an event that has not ended is reported as an error)
   SplitRegion& r = g_split_region[dev][pick];
   if (r.used && hipStreamWaitEvent(st, r.done, 0) != hipSuccess) return nullptr;
   *out = &r;

@@ -17,8 +17,9 @@
 // Launch shape: align (1 WG) -> gemm1 (+silu*up) -> gemm2 (*w) -> combine,
 // grid-stride kernels over a plan in global memory; the align launch is
 // skipped when the caller hands in the plan its router-split gap kernel
-// built.  Calls with many tokens per expert (prefill chunks) run the tiled
-// product of tile.h instead.  (A single persistent kernel with cross-workgroup hand-offs was
+// built, and in small calls, whose gemm1 groups the pairs itself.  Calls with
+// many tokens per expert (prefill chunks) run the tiled product of tile.h
+// instead.  (A single persistent kernel with cross-workgroup hand-offs was
 // measured 1.6-1.8x slower than these launches and is not kept.)
 #include <math.h>
 
@@ -1131,21 +1132,27 @@ struct TileFor<false, G1, 128> {
 // 244 at 128 (V2-Lite); fp8 32 / 64 pairs 592 / 637 at 16, 672 / 657 at 24.
 //
 // A call over few slots must also fill the device: the tiles are taken where
-// they make at least one item per CU.
+// they make at least one item per CU.  And a lane's offsets into the tokens
+// and into one expert's or the shared weights are 32-bit.
 template <bool FP8>
-int tile_pairs(const CallShape& cs, int E, int S) {
+int tile_pairs(const CallShape& cs, int E, int S, int shared_I) {
   const int slots = std::min(E, S), P = cs.T * cs.k;
+  const size_t rows = std::max<size_t>(cs.T, std::max<size_t>(2 * cs.I, 2 * (size_t)shared_I));
+  if (rows * cs.H * 2 > UINT32_MAX) return 0;
   if (P <= SLUICE_MAX_PAIRS && P < (FP8 ? 6 : 10) * slots) return 0;
   const int bm = FP8 ? (P < 20 * slots ? 32 : 64) : P < 64 * slots ? 64 : 128;
-  const int rows = bm == 128 ? 256 : 128;
-  const long items = (long)std::max(P / bm, slots) * std::min(2 * cs.I / rows, cs.H / rows);
+  const int ch = bm == 128 ? 256 : 128;
+  const long items = (long)std::max(P / bm, slots) * std::min(2 * cs.I / ch, cs.H / ch);
   return P > SLUICE_MAX_PAIRS || items >= 256 ? bm : 0;
 }
 
 // Workgroups of a persistent tile launch: as many as fit the device at once
-// (a multiple of 8: the XCDs), looked up once per device and kernel.
+// (a multiple of 8: the XCDs), looked up once per device and kernel.  Over a
+// map whose slots may stream, a CU's worth less per XCD: waiting workgroups
+// would else hold every CU's LDS, and the kernels that fill the slots (the
+// runtime's copy kernel, the decode of coded rows) must be able to start.
 template <typename C>
-int tile_grid(long items, int* out) {
+int tile_grid(long items, bool waits, int* out) {
   static std::atomic<int> cache[kWaitDevices];
   int dev = 0;
   SLUICE_HIP_CHECK(hipGetDevice(&dev));
@@ -1159,6 +1166,7 @@ int tile_grid(long items, int* out) {
     n = std::max(std::max(per_cu, 1) * std::max(cus, 1) / 8 * 8, 8);
     cache[dev].store(n, std::memory_order_relaxed);
   }
+  if (waits && n > 8) n -= std::min(n - 8, (n / 32 + 7) / 8 * 8);
   *out = (int)std::min<long>(n, (items + 7) / 8 * 8);
   return SLUICE_OK;
 }
@@ -1167,7 +1175,8 @@ template <typename C>
 int launch_tiles(const TileArgs& a, long tiles, hipStream_t st) {
   const int n_out = C::G1 ? a.cs.I : a.cs.H;
   int grid = 0;
-  const int rc = tile_grid<C>(tiles * ((n_out + C::kOut - 1) / C::kOut), &grid);
+  const int rc = tile_grid<C>(tiles * ((n_out + C::kOut - 1) / C::kOut),
+                              a.W.wait.pending != nullptr, &grid);
   if (rc != SLUICE_OK) return rc;
   hipLaunchKernelGGL(moe_tile_kernel<C>, dim3(grid), dim3(64 * C::NW), 0, st, a);
   return (int)hipGetLastError();
@@ -1196,7 +1205,9 @@ int run_tiled(const void* x, const ExpertW& W, const float* tw, const int32_t* t
   pl.valid = (int32_t*)(pl.tiles + tiles);
   pl.order = (uint16_t*)(pl.valid + (P + 3) / 4 * 4);
   if ((size_t)(pl.order + P2 - (uint16_t*)w.plan) > 2 * plan_ints(P)) return SLUICE_E_INVAL;
-  auto sort = P <= 8 * kSortThreads ? moe_sort_kernel<8> : moe_sort_kernel<64>;
+  auto sort = P <= 8 * kSortThreads    ? moe_sort_kernel<8>
+              : P <= 32 * kSortThreads ? moe_sort_kernel<32>
+                                       : moe_sort_kernel<64>;
   static_assert(SLUICE_MAX_PREFILL_PAIRS <= 64 * kSortThreads, "sort registers");
   hipLaunchKernelGGL(sort, dim3(1), dim3(kSortThreads), 0, st, ti, P, map, E, S, W.wait.pending, T,
                      n_sh, bm, pl);
@@ -1223,7 +1234,7 @@ int run_experts(const void* x, const ExpertW& W, const float* tw, const int32_t*
   const CallShape cs{T, k, H, I};
   ExpertW Ww = W;
   if (map != nullptr) Ww.wait = slotwait_lookup(map);
-  const int bm = plan == nullptr ? tile_pairs<FP8>(cs, E, S) : 0;
+  const int bm = plan == nullptr ? tile_pairs<FP8>(cs, E, S, Ww.I_s) : 0;
   if (bm > 0)
     return run_tiled<FP8>(x, Ww, tw, ti, map, cs, E, S, n_sh, bm, scale, shared, w, out, st);
   const bool self = plan == nullptr && Ww.wait.pending == nullptr && P <= kSelfPairs;

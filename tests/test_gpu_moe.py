@@ -434,7 +434,8 @@ ONE_ROUNDING = 2.0 ** -8
     (500, 1152, 640, 640, 48, 48, 4, 1.0, True),    # fp8, 64-pair tiles
     (1100, 1152, 640, 0, 64, 48, 4, 0.8, True),     # fp8, over 4096 pairs
     (96, 9216, 1024, 0, 40, 32, 4, 1.0, True),      # over 64 scale chunks of K
-    (1700, 512, 256, 0, 64, 64, 5, 1.0, False),     # over 8192 pairs: the sort's larger form
+    (1700, 512, 256, 0, 64, 64, 5, 1.0, False),     # over 8192 pairs: the sort's next form
+    (4200, 64, 64, 0, 64, 64, 8, 0.9, False),       # over 32768 pairs: its largest
 ])
 def test_tiled_product_matches_the_decode_kernels(T, H, I, Is, E, S, k, frac, fp8):
     from sluice_amd import ops
