@@ -932,6 +932,13 @@ constexpr int kMaxShared = 4;
 // partial bytes of a call above which the combine reads valid words first
 constexpr long kCombineCheckFirstBytes = 2L << 20;
 
+// w * v, rounded (not fused into the sum it joins: the decode kernels store
+// this product).
+__device__ __forceinline__ f32x4_t weighted(float w, f32x4_t v) {
+#pragma clang fp contract(off)
+  return w * v;
+}
+
 template <bool SPEC>
 __device__ __forceinline__ void combine4(const float* __restrict__ partial,
                                          const int32_t* __restrict__ valid,
@@ -960,7 +967,7 @@ __device__ __forceinline__ void combine4(const float* __restrict__ partial,
   f32x4_t acc = zero, acs = zero;
 #pragma unroll
   for (int j = 0; j < SLUICE_MAX_TOPK; ++j)
-    if (ok[j]) acc += topk_w != nullptr ? topk_w[t * k + j] * v[j] : v[j];
+    if (ok[j]) acc += topk_w != nullptr ? weighted(topk_w[t * k + j], v[j]) : v[j];
 #pragma unroll
   for (int u = 0; u < kMaxShared; ++u)
     if (u < n_sh) acs += vs[u];

@@ -16,24 +16,35 @@
 //   * gemm2: partial[pair] = W2 . act[pos] (fp32), which the combine weights
 //     and sums.
 //
+// A pair's sums have the decode kernels' order, so its bits depend neither on
+// the size of its call nor on the slot its expert sits in: the products of a
+// chunk meet in the same MFMAs, and K is summed in the decode kernels' parts
+// (their waves), whose sums are added in part order.  The parts cost a second
+// set of accumulators.  (K in one sum, started at an offset of the slot's own
+// so that workgroups do not meet in the same memory channels, measured 216
+// against 226, 574 against 593 and 696 against 705 us for the calls below.)
+//
 // Bound: HBM while the experts have few tokens (the weights are read once;
 // 4.9 TB/s in gemm1 of the V2-Lite call below, the DMA stream alone reaches
 // 6.2), the operand traffic out of L2 beyond (a 4096-token call runs no faster
-// with the LDS reads scheduled between the products).  Whole calls against the
-// decode kernels: Qwen3 shape, 4096 tokens, 4084 -> 570 us; V2-Lite
-// shape, 509 tokens over 48 slots, 628 -> 229 us; V3 fp8, 384 tokens over 64 of
-// 256 experts, 1493 -> 717 us (rows past a tile's pairs not loaded, and fp8
-// widened to bf16 by one instruction per pair: 725 -> 698 side by side).
+// with the LDS reads scheduled between the products).  Whole calls, timed in
+// turn with the decode kernels, same bits: Qwen3 shape, 4096 tokens, 4076 ->
+// 593 us; V2-Lite shape, 509 tokens over 48 slots, 562 -> 225 us; V3 fp8, 384
+// tokens over 64 of 256 experts, 1438 -> 700 us (before rows past a tile's
+// pairs were left out and fp8 went to bf16 by one instruction per pair, 27 us
+// more).
 //
-// LDS rows are 128 bytes (64 bf16 or 128 fp8 of K) in eight 16-byte
-// segments, segment s of row r at s ^ (r & 7); the swizzle is in the lanes'
-// global addresses, since a DMA writes its lanes consecutively.  A 16-byte
-// LDS read serves 16 lanes at a time over 64 banks, and the lanes that meet
-// come from two neighbouring K groups (lanes 0-3, 12-15 and 20-27, ...): the
-// K groups of one read take neighbouring segments (4m + kb), so that the two
-// groups fall on even and odd segments (with segments 2kb + m half of the
-// LDS cycles were conflicts).  The fp8 product's token segments are stored in
-// the order its 16-value weight segments take them.
+// LDS rows are 128 bytes (64 bf16 or 128 fp8 of K) in eight 16-byte segments,
+// the segment at place p of row r stored at p ^ (r & 7); places and swizzle
+// are in the lanes' global addresses, since a DMA writes its lanes
+// consecutively.  A 16-byte LDS read serves 16 lanes at a time over 64 banks,
+// and the lanes that meet come from two neighbouring K groups (lanes 0-3,
+// 12-15 and 20-27, ...).  Read m of K group kb takes segment 2kb + m (the
+// decode kernels' order), which sits at place 4m + kb: the two groups then
+// fall on even and odd places (at place 2kb + m half of the LDS cycles were
+// conflicts).  An fp8 chunk's tokens are two rows of 64: half h of weight
+// segment 2kb + i meets token segment 4kb + 2i + h, place 4i + 2h + (kb & 1)
+// of row kb >> 1.
 //
 // (Internal to moe.hip, which includes it inside its anonymous namespace.)
 #pragma once
@@ -220,6 +231,7 @@ struct TileCfg {
   static constexpr int NW = WC * WP, ESZ = FP8 ? 1 : 2;
   static constexpr int KS = FP8 ? 128 : 64;       // K per stage
   static constexpr int SUB = KS / 64;             // 128-byte token sub-tiles per stage
+  static constexpr int KP = G1 ? kKS : G2Shape<FP8>::K;  // K parts, as the decode kernels have
   static constexpr int CW = CH / WC, PW = BM / WP;
   static constexpr int FM = CW / 16, FN = PW / 16;
   static constexpr int kStage = CH * 128 + BM * KS * 2;
@@ -261,8 +273,9 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
   const int per_xcd = (int)gridDim.x / xcds;
   const int r0 = (int)((long)routed * xcd / xcds), rn = (int)((long)routed * (xcd + 1) / xcds) - r0;
   const int s0 = (int)((long)shared * xcd / xcds), sn = (int)((long)shared * (xcd + 1) / xcds) - s0;
-  const int seg = (lane & 7) ^ (lane >> 3);
-  const int bseg = FP8 ? 2 * (seg & 3) + (seg >> 2) : seg;  // token segment of this lane
+  const int sp = (lane & 7) ^ (lane >> 3);            // LDS place of this lane's segment
+  const int aseg = 2 * (sp & 3) + (sp >> 2);          // weight segment there
+  const int bseg = FP8 ? (sp >> 1) + 4 * (sp & 1) : aseg;  // token segment
 
   struct Item {
     int slot_field, pos0, count, cb;
@@ -297,10 +310,6 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
     }
   };
 
-  // An item's first chunk: see issue.
-  auto first_chunk = [&](const Item& t) {
-    return (int)((unsigned)(3 * (t.slot_field & kSlotMask)) % (unsigned)nk);
-  };
   // The wave's fp8 block scales of an item, the 64 chunks of window w, chunk
   // c in lane c & 63 (a load per chunk would wait for every DMA in flight):
   // of its gate and up rows, or of its hidden rows.
@@ -323,7 +332,6 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
   // Operand addresses of the item being loaded.
   const uint8_t *abase = nullptr, *bbase = nullptr;
   uint32_t va[C::NA], vb[C::NB];
-  int k0 = 0;
   auto address = [&](const Item& it, const int (&rows)[C::NB]) {
     const int slot = it.slot_field & kSlotMask, ch0 = it.cb * C::kOut;
     uint32_t ald;
@@ -350,7 +358,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
       } else {
         row = (uint32_t)min(ch0 + l, H - 1);
       }
-      va[i] = row * ald + (uint32_t)seg * 16;
+      va[i] = row * ald + (uint32_t)aseg * 16;
     }
 #pragma unroll
     for (int i = 0; i < C::NB; ++i) {
@@ -361,17 +369,11 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
                            : row;
       vb[i] = row * (uint32_t)(K * 2) + (uint32_t)(token_sub(i) * 128 + bseg * 16);
     }
-    k0 = first_chunk(it);
   };
-  // Chunk k of the item goes to stage buffer buf.  The chunks are taken from
-  // k0 on, around the end: rows are a power of two apart in many models, and
-  // workgroups that all read the same columns meet in the same memory
-  // channels.  (k0 depends on the weights alone, so a pair's sum has one
-  // order whichever tile it lands in.)
+  // Chunk k of the item goes to stage buffer buf.
   auto issue = [&](int k, int buf, int nb) {
-    const int kk = k + k0 < nk ? k + k0 : k + k0 - nk;
-    const uint8_t* ap = abase + (size_t)kk * 128;
-    const uint8_t* bp = bbase + (size_t)kk * (C::KS * 2);
+    const uint8_t* ap = abase + (size_t)k * 128;
+    const uint8_t* bp = bbase + (size_t)k * (C::KS * 2);
     const uint32_t d = lds0 + (uint32_t)(buf * C::kStage);
 #pragma unroll
     for (int i = 0; i < C::NA; ++i) dma16(d + (wave + i * NW) * 1024, ap, va[i]);
@@ -393,7 +395,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
   int rows[C::NB];
   rows_of(it, rows);
   Scales nsc = {0.f, 0.f};
-  if (FP8) nsc = scales_of(it, first_chunk(it) >> 6);
+  if (FP8) nsc = scales_of(it, 0);
   await_slot(a.W.wait, it.slot_field);
   address(it, rows);
   issue_first(it.count);
@@ -402,10 +404,8 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
     const bool more = next < rn + sn;
     const Item nit = more ? item_at(next) : it;
     rows_of(nit, rows);
-    const int kf = k0;
     Scales sc = nsc;
-    int window = kf >> 6;
-    if (FP8) nsc = scales_of(nit, first_chunk(nit) >> 6);
+    if (FP8) nsc = scales_of(nit, 0);
     const int count = it.count, pos0 = it.pos0, ch0 = it.cb * C::kOut;
     const int wrow = G1 ? ch0 + wc * (C::CW / 2) : ch0 + wc * C::CW;  // the wave's first channel
     int pair[FN];  // this lane's (gemm2), for the epilogue
@@ -414,17 +414,28 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
       for (int g = 0; g < FN; ++g)
         pair[g] = a.plan.order[pos0 + min((g * C::WP + wp) * 16 + R, count - 1)];
     }
-    f32x4_t acc[FM][FN];
+    // tot: the sums of the K parts done, acc: the part being summed.
+    f32x4_t acc[FM][FN], tot[FM][FN];
 #pragma unroll
     for (int f = 0; f < FM; ++f)
 #pragma unroll
-      for (int g = 0; g < FN; ++g) acc[f][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      for (int g = 0; g < FN; ++g) tot[f][g] = acc[f][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     // The K loop over NG of the wave's FN token fragments: the fragments past
     // the tile's pairs are left out.
     const auto k_loop = [&](auto ng) {
       constexpr int NG = decltype(ng)::value;
-      int buf = 0;
+      int buf = 0, part = 1, cut = nk / C::KP;  // the next part and its first chunk
       for (int k = 0; k < nk; ++k) {
+        if (k == cut) {
+#pragma unroll
+          for (int f = 0; f < FM; ++f)
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+              tot[f][g] += acc[f][g];
+              acc[f][g] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            }
+          while (cut <= k) cut = ++part * nk / C::KP;
+        }
         constexpr int nb = C::loads(NG), L = C::NA + nb;
         const int ahead = min(ST - 2, nk - 1 - k);  // stages after k in flight
         if (ST >= 4 && ahead >= 2)
@@ -452,15 +463,11 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
               for (int g = 0; g < NG; ++g) acc[f][g] = mfma16x16x32_bf16(av[f], bv[g], acc[f][g]);
           }
         } else {
-          const int kk = k + kf < nk ? k + kf : k + kf - nk;
-          if (kk >> 6 != window) {
-            window = kk >> 6;
-            sc = scales_of(it, window);
-          }
+          if (k != 0 && (k & 63) == 0) sc = scales_of(it, k >> 6);
           const float c0 = __uint_as_float(
-              (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(sc.a), kk & 63));
+              (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(sc.a), k & 63));
           const float c1 = __uint_as_float(
-              (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(sc.b), kk & 63));
+              (uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(sc.b), k & 63));
           f32x4_t t[FM][NG];
 #pragma unroll
           for (int f = 0; f < FM; ++f)
@@ -475,7 +482,8 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
               fp8x16_to_bf16(ldl(sa + f * 2048 + oa), av[f][0], av[f][1]);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-              const int ob = ((4 * h + kb) ^ (R & 7)) * 16 + i * BM * 128;
+              const int ob =
+                  ((4 * i + 2 * h + (kb & 1)) ^ (R & 7)) * 16 + (kb >> 1) * (BM * 128);
               u32x4_t bv[NG];
 #pragma unroll
               for (int g = 0; g < NG; ++g) bv[g] = ldl(sb + g * C::WP * 2048 + ob);
@@ -519,7 +527,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
 #pragma unroll
         for (int f = 0; f < FM / 2; ++f) {
           const int ch = wrow + f * 16 + kb * 4;
-          const f32x4_t gt = acc[f][g], u = acc[f + FM / 2][g];
+          const f32x4_t gt = tot[f][g] + acc[f][g], u = tot[f + FM / 2][g] + acc[f + FM / 2][g];
           float o[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) o[r] = gt[r] / (1.0f + expf(-gt[r])) * u[r];
@@ -532,7 +540,8 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
         for (int f = 0; f < FM; ++f) {
           const int ch = wrow + f * 16 + kb * 4;
           if (ch < H)
-            *reinterpret_cast<f32x4_t*>(a.partial + (size_t)pair[g] * H + ch) = acc[f][g];
+            *reinterpret_cast<f32x4_t*>(a.partial + (size_t)pair[g] * H + ch) =
+                tot[f][g] + acc[f][g];
         }
       }
     }
