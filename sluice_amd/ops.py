@@ -98,10 +98,16 @@ def _(router_logits, top_k, scoring="softmax", renormalize=False, routed_scaling
 # ---------------------------------------------------------------------------
 # Expert product
 # ---------------------------------------------------------------------------
+def _index(device: torch.device) -> int:
+    return device.index if device.index is not None else torch.cuda.current_device()
+
+
 class _Workspace:
     """One grow-only device workspace per device, shared by every layer (the
     layers run one after another on one stream).  reserve() sizes it ahead of
-    graph capture so captured launches bake a pointer that never moves.
+    graph capture.  Captured launches bake the buffer's address, so a buffer
+    that was handed out during a capture is kept when a larger one takes its
+    place.
     ``zero``: the buffer is zero-filled when (re)allocated, for kernels that
     keep counters in it; the expert product's workspace needs no initial
     contents."""
@@ -109,27 +115,36 @@ class _Workspace:
     def __init__(self, zero: bool = False):
         self.buf: dict[int, torch.Tensor] = {}
         self.zero = zero
+        self.captured: set[int] = set()       # devices whose current buffer a graph has baked
+        self.kept: list[torch.Tensor] = []    # replaced buffers that graphs have baked
 
     def get(self, device: torch.device, nbytes: int) -> torch.Tensor:
-        idx = device.index if device.index is not None else torch.cuda.current_device()
+        idx = _index(device)
         cur = self.buf.get(idx)
+        capturing = torch.cuda.is_current_stream_capturing()
         if cur is None or cur.numel() < nbytes:
-            if torch.cuda.is_current_stream_capturing():
+            if capturing:
                 raise RuntimeError(
                     "sluice fused_experts workspace too small during graph capture; call "
                     "sluice_amd.ops.reserve_workspace(...) before capturing")
             alloc = torch.zeros if self.zero else torch.empty
-            cur = alloc(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-            self.buf[idx] = cur
+            new = alloc(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
+            if idx in self.captured:
+                self.kept.append(cur)
+                self.captured.discard(idx)
+            self.buf[idx] = cur = new
+        if capturing:
+            self.captured.add(idx)
         return cur
 
     def size(self, device: torch.device) -> int:
-        idx = device.index if device.index is not None else torch.cuda.current_device()
-        cur = self.buf.get(idx)
+        cur = self.buf.get(_index(device))
         return 0 if cur is None else cur.numel()
 
 
 _WS = _Workspace()
+# device -> the smallest prefill workspace that could not be allocated there
+_PREFILL_OOM: dict[int, int] = {}
 
 
 def workspace_bytes(T: int, H: int, I: int, k: int, shared_I: int = 0) -> int:
@@ -220,8 +235,10 @@ def _fused_experts_impl(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch
     # More (token, expert) pairs than one launch takes (a prefill chunk on the
     # classic path): tokens are independent, so run slices of them, as few as
     # the prefill entry's bounds allow.
-    step = T if T <= chunk else _prefill_slice(T, H, I, k, Is, chunk, x.device)
-    ws = _WS.get(x.device, workspace_bytes(min(T, step), H, I, k, Is))
+    if T <= chunk:
+        step, ws = T, _WS.get(x.device, workspace_bytes(T, H, I, k, Is))
+    else:
+        step, ws = _prefill_workspace(T, H, I, k, Is, chunk, x.device)
     for t0 in range(0, T, step):
         n = min(step, T - t0)
         row = 2 * H * t0
@@ -253,23 +270,39 @@ def _fused_experts_impl(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch
     return out
 
 
-def _prefill_slice(T: int, H: int, I: int, k: int, Is: int, chunk: int, device) -> int:
-    """Tokens per launch of a call of more than ``chunk`` tokens: equal slices
-    within the prefill entry's pair and workspace bounds, or ``chunk`` where
-    the workspace cannot grow to that: while a graph is being captured, or
-    without the memory for it."""
+def _prefill_workspace(T: int, H: int, I: int, k: int, Is: int, chunk: int, device):
+    """(tokens per launch, workspace) of a call of more than ``chunk`` tokens:
+    equal slices within the prefill entry's pair and workspace bounds, over the
+    shared workspace where one that large was reserved and over memory of the
+    call's own (torch's caching allocator, given back when the call returns)
+    otherwise: the shared one never grows for speed, since other programs'
+    memory and captured graphs' addresses hang on it.  While a graph is
+    captured, or without the memory, slices of ``chunk`` over the shared one."""
     per = workspace_bytes(_MAX_PAIRS, H, I, k, Is) // _MAX_PAIRS + 1
     most = max(chunk, min(_MAX_PREFILL_PAIRS // (k + Is // I), _MAX_PREFILL_WORKSPACE // per))
     step = -(-T // -(-T // most))
     need = workspace_bytes(step, H, I, k, Is)
-    if _WS.size(device) < need:
-        if torch.cuda.is_current_stream_capturing():
-            return chunk
+    if _WS.size(device) >= need:
+        return step, _WS.get(device, need)
+    if not torch.cuda.is_current_stream_capturing() and _may_allocate(device, need):
+        idx = _index(device)
         try:
-            _WS.get(device, need)
+            ws = torch.empty(need, dtype=torch.uint8, device=device)
+            _PREFILL_OOM.pop(idx, None)
+            return step, ws
         except torch.OutOfMemoryError:
-            return chunk
-    return step
+            _PREFILL_OOM[idx] = need
+    return chunk, _WS.get(device, workspace_bytes(chunk, H, I, k, Is))
+
+
+def _may_allocate(device, need: int) -> bool:
+    """False while memory that was out for a smaller or equal workspace is
+    still short: a failed allocation makes torch give back its whole cache, so
+    it is not tried on each call."""
+    if need < _PREFILL_OOM.get(_index(device), need + 1):
+        return True
+    cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+    return torch.cuda.mem_get_info(device)[0] + cached >= need
 
 
 @torch.library.custom_op("sluice::fused_experts", mutates_args=())

@@ -524,6 +524,34 @@ def test_prefill_slices_follow_the_reserved_workspace(monkeypatch):
         assert torch.equal(got, want)
 
 
+def test_graphs_replay_after_a_longer_eager_call(monkeypatch):
+    """A graph captured over the reserved workspace gives the eager bits after
+    an eager call that needs more than it holds, with the memory that this
+    call gave back written over."""
+    from sluice_amd import ops
+
+    args, kw = _tile_case(1000, 1088, 448, 0, 40, 40, 5, 0.8, False, seed=6)
+    short = [args[0][:5], args[1], args[2], args[3][:5], args[4][:5]]
+    monkeypatch.setattr(ops, "_WS", ops._Workspace())
+    ops.reserve_workspace(DEV, 5, 1088, 448, 5)
+    want, want_long = ops.fused_experts(*short, **kw), None
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = ops.fused_experts(*short, **kw)
+    for i in range(3):
+        long = ops.fused_experts(*args, **kw)
+        over = [torch.full((n,), float("nan"), device=DEV) for n in (1 << 18, 1 << 23)]
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        assert all(torch.isnan(t).all() for t in over)
+        assert want_long is None or torch.equal(long, want_long)
+        want_long = long
+        ops.fused_experts(args[0][:700], args[1], args[2], args[3][:700], args[4][:700], **kw)
+
+
 def test_tiled_product_over_a_map_whose_slots_streamed():
     """A prefill call over the map of a layer whose last gap filled slots
     waits for them like the decode kernels do, and gives their product."""
