@@ -394,9 +394,20 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
   Item it = item_at(n);
   int rows[C::NB];
   rows_of(it, rows);
+  // The first scales of the item loaded next: ahead of its weights, or, where
+  // the slot's rows may still stream, behind the wait like every other read
+  // of them (the gap kernel itself copies scale rows only up to 32 KB and in
+  // whole 16-byte vectors; others arrive with the weights).
   Scales nsc = {0.f, 0.f};
-  if (FP8) nsc = scales_of(it, 0);
-  await_slot(a.W.wait, it.slot_field);
+  auto scales_early = [&](const Item& t) {
+    if (FP8 && (t.slot_field & kPendingBit) == 0) nsc = scales_of(t, 0);
+  };
+  auto await_item = [&](const Item& t) {
+    await_slot(a.W.wait, t.slot_field);
+    if (FP8 && (t.slot_field & kPendingBit) != 0) nsc = scales_of(t, 0);
+  };
+  scales_early(it);
+  await_item(it);
   address(it, rows);
   issue_first(it.count);
   for (;;) {
@@ -405,7 +416,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
     const Item nit = more ? item_at(next) : it;
     rows_of(nit, rows);
     Scales sc = nsc;
-    if (FP8) nsc = scales_of(nit, 0);
+    scales_early(nit);
     const int count = it.count, pos0 = it.pos0, ch0 = it.cb * C::kOut;
     const int wrow = G1 ? ch0 + wc * (C::CW / 2) : ch0 + wc * C::CW;  // the wave's first channel
     int pair[FN];  // this lane's (gemm2), for the epilogue
@@ -513,7 +524,7 @@ __global__ __launch_bounds__(64 * C::NW) void moe_tile_kernel(TileArgs a) {
       k_loop(std::integral_constant<int, FN>{});
     if (more) {
       dma_wait<0>();  // every wave has read its last stage
-      await_slot(a.W.wait, nit.slot_field);
+      await_item(nit);
       address(nit, rows);
       issue_first(nit.count);
     }

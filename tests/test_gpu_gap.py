@@ -850,3 +850,63 @@ def test_wait_bound_set_after_capture_applies_to_replays(monkeypatch):
     for _ in range(4):
         served_step()
     off.close()
+
+
+@pytest.mark.parametrize("kind", ["bf16", "bf16-coded", "fp8"])
+def test_tiled_product_waits_for_rows_in_flight(monkeypatch, kind):
+    """A prefill call queued right behind a gap that fills every slot, while
+    the rows stream: its bits are those of a call over copies of the landed
+    rows and a map that no layer registered.  fp8: scale rows of 360 and 180
+    bytes, which arrive with the weights (the gap kernel copies none)."""
+    from sluice_amd import _lib, ops
+
+    E, S, k, H, I, T = 96, 32, 4, 1152, 640, 96
+    print(f"tiles over rows in flight: {kind}", flush=True)
+    monkeypatch.setenv("SLUICE_STAGE_ROWS", "0")
+    monkeypatch.setenv("SLUICE_CODEC", "1" if kind == "bf16-coded" else "0")
+    fp8 = kind == "fp8"
+    layer = _Fp8Layer(E, H, I) if fp8 else _Layer(E, E, H=H, I=I)
+    off = _offloader(monkeypatch, S, 0.0, False)
+    off.wrap_modules(iter([layer]))
+    with torch.cuda.device(DEV):
+        off.post_init()
+    cache = off._caches[id(layer)]
+    off._rs_caches.append(cache)
+    lib = _lib.load()
+    if fp8:
+        assert lib.sluice_layer_pulled_params(cache.handle) == 0
+    off.start_gap_server()
+    ops.reserve_workspace(DEV, T, H, I, k)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rng = np.random.default_rng(3)
+    x = (torch.randn((T, H), generator=g, device=DEV) * 0.1).to(torch.bfloat16)
+    tw = torch.rand((T, k), generator=g, device=DEV)
+    hs = torch.zeros((S // k, 64), dtype=torch.bfloat16, device=DEV)
+
+    def product(weights, emap, ids):
+        kw = dict(w1_scale=weights["w13_weight_scale"], w2_scale=weights["w2_weight_scale"],
+                  block_shape=[128, 128]) if fp8 else {}
+        return ops.fused_experts(x, weights["w13_weight"], weights["w2_weight"], tw, ids,
+                                 global_num_experts=E, expert_map=emap, **kw)
+
+    perm = rng.permutation(E).astype(np.int32).reshape(3, S)
+    assert lib.sluice_gap_set_timeout(5.0) == 0
+    try:
+        for n in range(6):
+            experts = perm[n % 3]
+            sel = torch.from_numpy(experts).to(DEV).view(-1, k)
+            ids = torch.from_numpy(rng.choice(experts, (T, k)).astype(np.int32)).to(DEV)
+            torch.cuda.synchronize()
+            torch.ops.vllm.sluice_stream_gap(hs, sel, 0)
+            got = product(cache.gpu_cache, cache.expert_map_buf, ids)
+            off.drain()
+            _slot_bytes_match_host(cache)
+            landed = {name: t.clone() for name, t in cache.gpu_cache.items()}
+            want = product(landed, cache.expert_map_buf.clone(), ids)
+            torch.cuda.synchronize()
+            assert (want != 0).any()
+            assert torch.equal(got, want), n
+        assert cache.stats()["misses"] >= 6 * S - S  # every slot refilled each time
+    finally:
+        lib.sluice_gap_set_timeout(0.0)
+        off.close()
