@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
 __device__ __forceinline__ void dma16(uint32_t lds, const void* base, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                ::"s"(lds), "v"(voff), "s"(base)
-               : "memory");
+               : "memory", "m0");
 }
 
 // Waits until at most N of this wave's DMAs are in flight and its LDS reads

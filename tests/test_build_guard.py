@@ -81,3 +81,20 @@ def test_decode_room_needs_the_decode_kernels_remarks():
 def test_decode_room_ignores_the_fp8_split_launch():
     # coded stores hold bf16 rows: decodes never wait beside the fp8 launch
     assert b.check_decode_room(_remarks(SPLIT, 112, 8, 4), _remarks(DECODE, 60, 0, 8)) == []
+
+
+def test_asm_that_writes_m0_names_it():
+    """The compiler keeps values of its own in m0: inline assembly that writes
+    it must list it as clobbered."""
+    import os
+    import re
+
+    seen = 0
+    for name in sorted(os.listdir(b.CSRC)):
+        with open(os.path.join(b.CSRC, name)) as f:
+            text = f.read()
+        for m in re.finditer(r"\basm\b[^;]*?;", text, re.S):
+            if re.search(r"\bs_mov_b32 m0\b", m.group(0)):
+                seen += 1
+                assert '"m0"' in m.group(0), (name, m.group(0))
+    assert seen > 0
