@@ -187,11 +187,14 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
 // register is written, so the compiler has nothing to reuse early; the
 // matching wait is dma_wait.  (With the builtin the compiler waits for every
 // DMA in flight at each LDS read.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved; its own uses see the clobber
 __device__ __forceinline__ void dma16(uint32_t lds, const void* base, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                ::"s"(lds), "v"(voff), "s"(base)
                : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 // Waits until at most N of this wave's DMAs are in flight and its LDS reads
 // are done, then for the whole workgroup.
