@@ -1057,7 +1057,9 @@ __global__ __launch_bounds__(WAVES * 64) void gqa_decode_kernel(
 // are the A operand of O[head][column] = P . V in the K order of mla_kpos;
 // V's operand (8 rows of one column per lane) is put together from 16-byte
 // row loads by byte permutes, 8 columns per lane.  P stays fp32: it enters
-// the product as three bf16 terms whose sum is P exactly.  One step's rows in
+// the product as three bf16 terms whose sum is P exactly.  The first two are
+// taken from the value just below, so that no term of a P > 0 is 0 and an
+// infinity in V stays one (0 x Inf would be NaN).  One step's rows in
 // registers per wave and three waves per SIMD (a second step in flight at two
 // waves per SIMD measured the same).  Qwen3 heads (32 over 4), against the
 // one-launch kernel above: 36.5 -> 11.0 us for one sequence of 4000 rows, 45.6
@@ -1210,7 +1212,7 @@ __global__ __launch_bounds__(kSplitWaves * 64, 3) void gqa_split_kernel(
     const float ref = mn == -INFINITY ? 0.f : mn;
     const float f = __builtin_amdgcn_exp2f(m - ref);
     float ps = 0.f;
-    u32x4_t pa[3];  // P as three bf16 terms, each the top 16 bits of what is left
+    u32x4_t pa[3];  // P as three bf16 terms: the top 16 bits of (just below) what is left
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       pv[j] = __builtin_amdgcn_exp2f(pv[j] - ref);
@@ -1220,7 +1222,9 @@ __global__ __launch_bounds__(kSplitWaves * 64, 3) void gqa_split_kernel(
     for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int j = 0; j < 8; j += 2) {
-        const uint32_t a = __float_as_uint(pv[j]), e = __float_as_uint(pv[j + 1]);
+        const uint32_t below = c < 2 ? 1u : 0u;  // of 0: 0
+        const uint32_t a = __builtin_elementwise_sub_sat(__float_as_uint(pv[j]), below);
+        const uint32_t e = __builtin_elementwise_sub_sat(__float_as_uint(pv[j + 1]), below);
         pa[c][j / 2] = __builtin_amdgcn_perm(e, a, 0x07060302u);
         pv[j] -= __uint_as_float(a & 0xffff0000u);
         pv[j + 1] -= __uint_as_float(e & 0xffff0000u);

@@ -489,6 +489,52 @@ def test_gqa_decode_split_matches_the_one_launch_kernel(nh, kvh, L, parts):
         assert torch.isnan(k1[t, :, p + 1:]).all() and torch.equal(k1[t, :, :p], k[t, :, :p])
 
 
+def test_gqa_decode_split_keeps_infinities():
+    """An infinity in a column of V gives what the one-launch kernel gives: an
+    infinity of its sign in that column (whatever the weight of its row, 1
+    among them), NaN where both signs meet, the finite columns as they are."""
+    lib, check = _lib()
+    c, nh, kvh, hd, L = 4, 32, 4, 128, 1024
+    inf = float("inf")
+    g = torch.Generator(device=DEV).manual_seed(77)
+
+    def rand(shape):
+        return torch.randn(shape, generator=g, device=DEV).bfloat16()
+
+    qkv, k, v = rand((c, (nh + 2 * kvh) * hd)), rand((c, kvh, L, hd)), rand((c, kvh, L, hd))
+    pos = torch.tensor([1000, 900, 800, 1023], device=DEV)
+    k[3] = 0          # scores of 0: every weight of token 3 is 1 before the sum
+    v[0, 1, 17, 5] = inf
+    v[1, 2, 128:640, 7] = -inf  # a wave's highest score among them
+    v[2, 0, 40, 9], v[2, 0, 700, 9] = inf, -inf
+    v[3, 3, 5, 100] = inf
+    w = torch.ones(hd, dtype=torch.bfloat16, device=DEV)
+    cos_t, sin_t = (a.to(DEV) for a in _tables(L, hd, 1e6))
+
+    def call(k, v, out):
+        check(lib.sluice_dec_gqa_decode(
+            qkv.data_ptr(), None, 0, w.data_ptr(), w.data_ptr(), cos_t.data_ptr(),
+            sin_t.data_ptr(), pos.data_ptr(), c, nh, kvh, hd, L, 1e-6, hd ** -0.5, k.data_ptr(),
+            v.data_ptr(), out.data_ptr(), _st()), "gqa_decode")
+
+    got, ref = (torch.empty((c, nh * hd), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    call(k.clone(), v.clone(), got)
+    k2, v2 = k.clone(), v.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()  # a captured call runs the one-launch kernel
+    with torch.cuda.graph(graph):
+        call(k2, v2, ref)
+    graph.replay()
+    torch.cuda.synchronize()
+    got, ref = got.float().cpu(), ref.float().cpu()
+    assert torch.isinf(ref).sum() == 3 * 8 and torch.isnan(ref).sum() == 8
+    assert torch.equal(torch.isnan(got), torch.isnan(ref))
+    assert torch.equal(got[torch.isinf(ref)], ref[torch.isinf(ref)])
+    fin = torch.isfinite(ref)
+    assert torch.isfinite(got[fin]).all()
+    assert _rel(got[fin], ref[fin]) <= 2.0 ** -8
+
+
 def test_gqa_decode_split_on_more_streams_than_scratch_regions():
     """Calls in flight on more streams than there are scratch regions give the
     bits they give one after another."""
