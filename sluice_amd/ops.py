@@ -336,8 +336,10 @@ def _(hidden_states, w1, w2, topk_weights, topk_ids, activation="silu", global_n
 
 def _nothing_watches(tensors) -> bool:
     """No transform, mode, tracer, profiler or gradient would see an op called
-    on these arguments: the op then does nothing but call its body."""
+    on these arguments, and none of them is a lazy view that its dispatch would
+    resolve: the op then does nothing but call its body."""
     if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack()
+            or torch._C._len_torch_function_stack()
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch._C._get_tracing_state() is not None
             or torch.autograd._profiler_enabled()
@@ -350,6 +352,8 @@ def _nothing_watches(tensors) -> bool:
         if type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter:
             return False
         if t.device.type != "cuda" or (grad and t.requires_grad):
+            return False
+        if t.is_neg() or t.is_conj() or t._is_zerotensor():
             return False
     return True
 

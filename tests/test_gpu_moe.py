@@ -611,6 +611,34 @@ def test_fused_experts_goes_through_the_op_when_something_watches():
         ops.fused_experts(*args, **kw, no_such_argument=1)
 
 
+def test_function_modes_and_lazy_views_go_through_the_op():
+    """A torch-function mode sees the op; routing weights that are lazily
+    negated or lazily zero have their values."""
+    from torch.overrides import TorchFunctionMode
+
+    from sluice_amd import ops
+
+    args, kw = _tile_case(3, 256, 64, 0, 8, 8, 2, 1.0, False, seed=8)
+    want = torch.ops.sluice.fused_experts(*args, **kw)
+    seen = []
+
+    class Watch(TorchFunctionMode):
+        def __torch_function__(self, func, types, a=(), k=None):
+            seen.append(str(func))
+            return func(*a, **(k or {}))
+
+    with Watch():
+        assert torch.equal(ops.fused_experts(*args, **kw), want)
+    assert any("fused_experts" in s for s in seen)
+    tw = args[3]
+    neg = torch.complex(tw, -tw).conj().imag
+    assert neg.is_neg() and torch.equal(neg, tw)
+    args[3] = neg
+    assert torch.equal(ops.fused_experts(*args, **kw), want)
+    args[3] = torch._efficientzerotensor(tw.shape, dtype=tw.dtype, device=DEV)
+    assert (ops.fused_experts(*args, **kw) == 0).all()
+
+
 @pytest.mark.parametrize("T,k,E,S,how", [
     (1, 1, 1, 1, "even"),          # one pair
     (1, 6, 64, 48, "even"),
