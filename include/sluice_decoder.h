@@ -125,10 +125,11 @@ int sluice_dec_mla_decode(const void* q, int q_stride, const void* kva, int kva_
  *   Exactly one of qkv and qkv_parts: the QKV projection's K parts
  *   [n_parts, c, (nh + 2*kvh)*hd] fp32 (n_parts <= 4, as sluice_dec_linear_split
  *   leaves them) are summed in order and rounded to bf16 first.
- *   Caches of more than 768 rows with several query heads per kv head run
- *   split over the rows in two launches over scratch of the library's own (26
- *   MB per GPU, held until the process ends), calls on any streams and threads
- *   kept apart by events; while the stream is captured, one launch. */
+ *   In caches of more than 768 rows with several query heads per kv head, a
+ *   token of more than 768 rows is split over them, in the same launch, over
+ *   scratch of the library's own (17 MB per GPU, held until the process ends;
+ *   calls on any streams and threads are kept apart).  While the stream is
+ *   captured, and for tokens of fewer rows, a workgroup takes a query head. */
 int sluice_dec_gqa_decode(const void* qkv, const float* qkv_parts, int n_parts,
                           const void* q_norm, const void* k_norm,
                           const float* cos_t, const float* sin_t, const int64_t* pos, int c,

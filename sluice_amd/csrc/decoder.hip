@@ -12,10 +12,13 @@
 #include "sluice_decoder.h"
 #include "stream.h"
 
-// Scratch of the split attention: see SplitRegion.
+// Scratch of the split attention (see SplitScratch): 512 workgroups' sums of 16
+// heads (528 bytes each) and their tickets, which are zero between launches.
 constexpr int kSplitRegions = 4;
-constexpr size_t kSplitRegionBytes = 13u << 19;  // 768 splits of 16 heads' 528-byte sums
+constexpr size_t kSplitRegionBytes = 512 * 16 * 528;
+constexpr int kSplitTickets = 512;
 static __device__ __align__(256) uint8_t split_scratch[kSplitRegions * kSplitRegionBytes];
+static __device__ int split_tickets[kSplitRegions * kSplitTickets];
 
 namespace {
 
@@ -911,19 +914,34 @@ __device__ __forceinline__ void gqa_chunk(const u32x4_t* kr, const u32x4_t* vr, 
 constexpr int kGqaWaves = 8;
 constexpr int kGqaRows = 2;
 
-template <int WAVES, int RG>
-__global__ __launch_bounds__(WAVES * 64) void gqa_decode_kernel(
-    const uint16_t* __restrict__ qkv, const float* __restrict__ qkv_parts, int nparts,
-    const uint16_t* __restrict__ q_norm,
-    const uint16_t* __restrict__ k_norm, const float* __restrict__ cos_t,
-    const float* __restrict__ sin_t, const int64_t* __restrict__ pos, int nh, int kvh, int L,
-    float eps, float scale, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
-    uint16_t* __restrict__ out) {
+// The arguments of the attention kernels, and their names.
+#define GQA_PARAMS                                                                            \
+  const uint16_t *__restrict__ qkv, const float *__restrict__ qkv_parts, int nparts,          \
+      const uint16_t *__restrict__ q_norm, const uint16_t *__restrict__ k_norm,               \
+      const float *__restrict__ cos_t, const float *__restrict__ sin_t,                       \
+      const int64_t *__restrict__ pos, int c, int nh, int kvh, int L, float eps, float scale, \
+      uint16_t *__restrict__ k_cache, uint16_t *__restrict__ v_cache, uint16_t *__restrict__ out
+#define GQA_ARGS                                                                               \
+  qkv, qkv_parts, nparts, q_norm, k_norm, cos_t, sin_t, pos, c, nh, kvh, L, eps, scale, k_cache, \
+      v_cache, out
+
+template <int WAVES>
+struct GqaLds {
+  float acc[WAVES * 4][kHd];
+  float m[WAVES * 4], l[WAVES * 4];
+};
+
+// Query head h of token t, one workgroup.  KNOWN: the caller has looked at the
+// position, which is in the cache, and no row past it is read (else the first
+// chunk's loads go out with the position's, and rows past it weigh 0).
+template <int WAVES, int RG, bool KNOWN>
+__device__ __forceinline__ void gqa_head(GQA_PARAMS, int t, int h, GqaLds<WAVES>& lds) {
   constexpr int NG = WAVES * 4;
   constexpr int CH = NG * RG;
-  __shared__ float gacc[NG][kHd];
-  __shared__ float gm[NG], gl[NG];
-  const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  auto& gacc = lds.acc;
+  auto& gm = lds.m;
+  auto& gl = lds.l;
+  const int tid = threadIdx.x;
   const int grp = nh / kvh, g = h / grp;
   const int sub = tid & 15, gi = tid >> 4;
   const int col = sub * 8;
@@ -944,7 +962,7 @@ __global__ __launch_bounds__(WAVES * 64) void gqa_decode_kernel(
     for (int v = 0; v < 3; ++v)
 #pragma unroll
       for (int q = 0; q < kMaxDeltaParts; ++q) {
-        const float* src = qkv_parts + ((size_t)(q < nparts ? q : 0) * gridDim.x + t) * width + offs[v];
+        const float* src = qkv_parts + ((size_t)(q < nparts ? q : 0) * c + t) * width + offs[v];
         pv[v][q][0] = *reinterpret_cast<const f32x4_t*>(src);
         pv[v][q][1] = *reinterpret_cast<const f32x4_t*>(src + 4);
       }
@@ -971,15 +989,19 @@ __global__ __launch_bounds__(WAVES * 64) void gqa_decode_kernel(
   }
   const u32x4_t wq = ldg16(q_norm + col), wk = ldg16(k_norm + col);
   u32x4_t kr[RG], vr[RG];
+  if (KNOWN) {
+    gqa_load_chunk<RG, NG>(k_cache, v_cache, cbase, 0, gi, (int)pos[t], kr, vr);
+  } else {
 #pragma unroll
-  for (int r = 0; r < RG; ++r) {
-    const int l = gi + NG * r;
-    const size_t off = (size_t)(l < L ? l : L - 1) * kHd;
-    kr[r] = ldg16(k_cache + cbase + off);
-    vr[r] = ldg16(v_cache + cbase + off);
+    for (int r = 0; r < RG; ++r) {
+      const int l = gi + NG * r;
+      const size_t off = (size_t)(l < L ? l : L - 1) * kHd;
+      kr[r] = ldg16(k_cache + cbase + off);
+      vr[r] = ldg16(v_cache + cbase + off);
+    }
   }
   const long long p = pos[t];
-  if (p < 0 || p >= L) return;
+  if (!KNOWN && (p < 0 || p >= L)) return;
   const int nc = (int)p;  // cache rows before the new one
   const int ci = (int)p * 64 + (sub & 7) * 8;
   float cs[8], sn[8];
@@ -1049,28 +1071,40 @@ __global__ __launch_bounds__(WAVES * 64) void gqa_decode_kernel(
   }
 }
 
-// The same for long caches, split over the rows, in two launches: a
-// workgroup takes one split of the rows for up to 16 query heads of one kv
-// head (a cache row is read once for all of them), the merge adds the splits
-// up.  On the matrix cores: a wave takes steps of 32 rows, scores
-// S^T[row][head] = K . q^T (two 16-row tiles, heads on N), whose registers
-// are the A operand of O[head][column] = P . V in the K order of mla_kpos;
-// V's operand (8 rows of one column per lane) is put together from 16-byte
-// row loads by byte permutes, 8 columns per lane.  P stays fp32: it enters
-// the product as three bf16 terms whose sum is P exactly.  The first two are
-// taken from the value just below, so that no term of a P > 0 is 0 and an
-// infinity in V stays one (0 x Inf would be NaN).  One step's rows in
-// registers per wave and three waves per SIMD (a second step in flight at two
-// waves per SIMD measured the same).  Qwen3 heads (32 over 4), against the
-// one-launch kernel above: 36.5 -> 11.0 us for one sequence of 4000 rows, 45.6
-// -> 17.5 for 12 of 700 to 4095 (72 MB: 4.1 TB/s), 12.4 -> 9.9 for 8 of 700
-// to 1023; the second launch loses below that, 6.9 -> 8.8 for 8 of 128 to 383.
-constexpr int kSplitWaves = 4;
+template <int WAVES, int RG>
+__global__ __launch_bounds__(WAVES * 64) void gqa_decode_kernel(GQA_PARAMS) {
+  __shared__ GqaLds<WAVES> lds;
+  gqa_head<WAVES, RG, false>(GQA_ARGS, blockIdx.x, blockIdx.y, lds);
+}
+
+// The same for long caches: a token of more than kSplitShort rows is split over
+// them, one of fewer runs as above, so that a cache's capacity costs a short
+// context nothing.  A workgroup takes one split of the rows for up to 16 query
+// heads of one kv head (a cache row is read once for all of them); the last one
+// of a token and kv head to finish adds the splits up.  On the matrix cores: a
+// wave takes steps of 32 rows, scores S^T[row][head] = K . q^T (two 16-row
+// tiles, heads on N), whose registers are the A operand of O[head][column] = P
+// . V in the K order of mla_kpos; V's operand (8 rows of one column per lane)
+// is put together from 16-byte row loads by byte permutes, 8 columns per lane.
+// P stays fp32: it enters the product as three bf16 terms whose sum is P
+// exactly.  The first two are taken from the value just below, so that no term
+// of a P > 0 is 0 and an infinity in V stays one (0 x Inf would be NaN).
+// Bound: the latency of a wave's dependent loads, hidden by 16 waves per CU (one
+// step's rows in registers each, 124 registers).
+constexpr int kSplitWaves = 8;
 constexpr int kSplitStep = 32;
 constexpr int kSplitHeads = 16;
 constexpr int kSplitMax = 16;         // splits per (token, kv head)
+constexpr int kSplitUnits = 512;      // workgroups that the splits of a call may make
 constexpr int kSplitQRow = kHd + 8;   // LDS row of one head's q (padded)
 constexpr int kSplitRec = kHd + 4;    // per (split, head): max, sum, -, -, O[128]
+// Qwen3 heads (32 over 4), eager calls one after another, the one-launch kernel
+// / this one with the line at 256 / 512 / 768 rows: 6.7 / 8.6 / 6.6 / 6.6 us
+// for 8 tokens of 128 to 383 rows, 8.8 / 9.0 / 8.8 / 8.7 for 8 of 384 to 767;
+// 10.6 / 9.3 for 8 of 700 to 1023, 42.3 / 19.0 for 12 of 700 to 4095 (72 MB),
+// 35.8 / 10.5 for one of 4000.  (Two launches, split and merge, behind events
+// that kept the streams apart: 11.1, 11.3, 11.5, 21.1 and 13.5 us.)
+constexpr int kSplitShort = 768;
 
 // Rows per split for n rows over `splits` of them: whole steps of every wave.
 __host__ __device__ inline int split_chunk(int n, int splits) {
@@ -1078,52 +1112,36 @@ __host__ __device__ inline int split_chunk(int n, int splits) {
   return ((n + splits - 1) / splits + kRound - 1) / kRound * kRound;
 }
 
-// grid (c * zh, kvh, splits), zh = ceil(query heads per kv head / 16).
-__global__ __launch_bounds__(kSplitWaves * 64, 3) void gqa_split_kernel(
-    const uint16_t* __restrict__ qkv, const float* __restrict__ qkv_parts, int nparts,
-    const uint16_t* __restrict__ q_norm, const uint16_t* __restrict__ k_norm,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
-    const int64_t* __restrict__ pos, int nh, int kvh, int zh, int L, float eps, float scale,
-    uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache, float* __restrict__ part) {
-  __shared__ __align__(16) uint16_t qs[(kSplitHeads + 2) * kSplitQRow];  // q, then new k and v
-  __shared__ __align__(16) float om[kSplitWaves][kSplitHeads][kHd];
-  __shared__ float ms[kSplitWaves][kSplitHeads], ls[kSplitWaves][kSplitHeads];
-  const int t = blockIdx.x / zh, z = blockIdx.x - t * zh, g = blockIdx.y, tid = threadIdx.x;
-  const int splits = gridDim.z, split = blockIdx.z;
-  const long long p = pos[t];
+// zh: groups of 16 query heads per kv head; tickets [c * zh * kvh], zero
+// between launches.
+struct SplitArgs {
+  int zh, splits;
+  float* part;
+  int* tickets;
+};
+
+struct SplitLds {
+  __align__(16) uint16_t qs[(kSplitHeads + 2) * kSplitQRow];  // q, then new k and v
+  __align__(16) float om[kSplitWaves][kSplitHeads][kHd];
+  float ms[kSplitWaves][kSplitHeads], ls[kSplitWaves][kSplitHeads];
+  int ticket;
+};
+
+// One split of token t's n rows for heads z * 16 .. of kv head g.
+__device__ __forceinline__ void gqa_part(GQA_PARAMS, const SplitArgs& sa, SplitLds& l, int t,
+                                         int z, int g, int split, int n) {
+  const int tid = threadIdx.x, splits = sa.splits;
+  const int chunk = split_chunk(n, splits);
+  const int r0 = split * chunk, r1 = min(n, r0 + chunk);
+  if (split >= splits || r0 >= n) return;
+  const int p = n - 1, last = max(p - 1, 0);
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int R = lane & 15, kb = lane >> 4;
   const int grp = nh / kvh, h0 = g * grp + z * kSplitHeads;
   const int heads = min(kSplitHeads, grp - z * kSplitHeads);
   const size_t cbase = ((size_t)t * kvh + g) * L * kHd;
-  const uint16_t* kc = k_cache + cbase;
-  const uint16_t* vc = v_cache + cbase;
-  // 16-lane group i takes vectors i and 16 + i: the query heads, then (16 and
-  // 17) the new k and v.
-  const int gi = tid >> 4, sub = tid & 15;
-  const size_t width = (size_t)(nh + 2 * kvh) * kHd;
-  auto load_vec = [&](int i) {
-    const int vec = (i < kSplitHeads ? h0 + min(i, heads - 1)
-                                     : nh + (i == kSplitHeads ? 0 : kvh) + g) * kHd + sub * 8;
-    if (qkv_parts == nullptr) return ldg16(qkv + t * width + vec);
-    // the projection's K parts: bf16(sum in part order)
-    f32x4_t a = {0.f, 0.f, 0.f, 0.f}, e = a;
-    for (int q = 0; q < nparts; ++q) {
-      const float* src = qkv_parts + ((size_t)q * (gridDim.x / zh) + t) * width + vec;
-      a += *reinterpret_cast<const f32x4_t*>(src);
-      e += *reinterpret_cast<const f32x4_t*>(src + 4);
-    }
-    return u32x4_t{pack2(a[0], a[1]), pack2(a[2], a[3]), pack2(e[0], e[1]), pack2(e[2], e[3])};
-  };
-  static_assert(kSplitWaves * 4 == kSplitHeads, "one query head per 16-lane group");
-  u32x4_t x = load_vec(gi), xn = {0u, 0u, 0u, 0u};
-  const u32x4_t wq = ldg16(q_norm + sub * 8), wk = ldg16(k_norm + sub * 8);
-  if (gi < 2) xn = load_vec(kSplitHeads + gi);
-  if (p < 0 || p >= L) return;
-  const int n = (int)p + 1, last = max((int)p - 1, 0);
-  const int chunk = split_chunk(n, splits);
-  const int r0 = split * chunk, r1 = min(n, r0 + chunk);
-  if (r0 >= n) return;
+  const uint8_t* kc = (const uint8_t*)(k_cache + cbase);
+  const uint8_t* vc = (const uint8_t*)(v_cache + cbase);
   // A step's operands: kr[u][m] = row 16u + R, columns 8 (4m + kb); vr[j] =
   // row (j < 4 ? 4kb + j : 16 + 4kb + j - 4), columns 8R.  (The new row is
   // taken from LDS: the cache's may not be written yet.)
@@ -1131,47 +1149,60 @@ __global__ __launch_bounds__(kSplitWaves * 64, 3) void gqa_split_kernel(
     u32x4_t kr[2][4], vr[8];
   };
   auto vrow = [&](int j) { return j < 4 ? 4 * kb + j : 12 + 4 * kb + j; };
-  auto load = [&](Step& s, int b) {
+  auto load_k = [&](Step& s, int b) {
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const uint16_t* r = kc + (size_t)min(b + 16 * u + R, last) * kHd + 8 * kb;
+      const uint32_t r = (uint32_t)min(b + 16 * u + R, last) * (2 * kHd) + 16 * kb;
 #pragma unroll
-      for (int m = 0; m < 4; ++m) s.kr[u][m] = ldg16(r + 32 * m);
+      for (int m = 0; m < 4; ++m) s.kr[u][m] = ldg16(kc + r + 64 * m);
     }
+  };
+  auto load_v = [&](Step& s, int b) {
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      s.vr[j] = ldg16(vc + (size_t)min(b + vrow(j), last) * kHd + 8 * R);
+      s.vr[j] = ldg16(vc + (uint32_t)min(b + vrow(j), last) * (2 * kHd) + 16 * R);
   };
   Step s0;
   const int b0 = r0 + w * kSplitStep;
-  if (b0 < r1) load(s0, b0);
-  {
-    const int ci = (int)p * 64 + (sub & 7) * 8;
-    float cs[8], sn[8], r[8];
-    *reinterpret_cast<f32x4_t*>(cs) = *reinterpret_cast<const f32x4_t*>(cos_t + ci);
-    *reinterpret_cast<f32x4_t*>(cs + 4) = *reinterpret_cast<const f32x4_t*>(cos_t + ci + 4);
-    *reinterpret_cast<f32x4_t*>(sn) = *reinterpret_cast<const f32x4_t*>(sin_t + ci);
-    *reinterpret_cast<f32x4_t*>(sn + 4) = *reinterpret_cast<const f32x4_t*>(sin_t + ci + 4);
-    auto rope = [&](u32x4_t v, u32x4_t wn) {
-      head_norm_rope(v, wn, cs, sn, eps, sub < 8, r);
-      return u32x4_t{pack2(r[0], r[1]), pack2(r[2], r[3]), pack2(r[4], r[5]), pack2(r[6], r[7])};
-    };
-    *reinterpret_cast<u32x4_t*>(&qs[gi * kSplitQRow + sub * 8]) = rope(x, wq);
-    if (gi < 2) {
-      if (gi == 0) xn = rope(xn, wk);
-      *reinterpret_cast<u32x4_t*>(&qs[(kSplitHeads + gi) * kSplitQRow + sub * 8]) = xn;
-      if (split == 0 && z == 0)
-        *reinterpret_cast<u32x4_t*>((gi == 0 ? k_cache : v_cache) + cbase + (size_t)p * kHd +
-                                    sub * 8) = xn;
+  if (b0 < r1) load_k(s0, b0);
+  // 16-lane group i: query head i; the new k (16) and v (17)
+  const int gi = tid >> 4, sub = tid & 15;
+  const size_t width = (size_t)(nh + 2 * kvh) * kHd;
+  if (gi < kSplitHeads + 2) {
+    const int vec = (gi < kSplitHeads ? h0 + min(gi, heads - 1)
+                                      : nh + (gi == kSplitHeads ? 0 : kvh) + g) * kHd + sub * 8;
+    u32x4_t x;
+    if (qkv_parts == nullptr) {
+      x = ldg16(qkv + t * width + vec);
+    } else {  // the projection's K parts: bf16(sum in part order)
+      f32x4_t a = {0.f, 0.f, 0.f, 0.f}, e = a;
+      for (int q = 0; q < nparts; ++q) {
+        const float* src = qkv_parts + ((size_t)q * c + t) * width + vec;
+        a += *reinterpret_cast<const f32x4_t*>(src);
+        e += *reinterpret_cast<const f32x4_t*>(src + 4);
+      }
+      x = u32x4_t{pack2(a[0], a[1]), pack2(a[2], a[3]), pack2(e[0], e[1]), pack2(e[2], e[3])};
     }
+    if (gi <= kSplitHeads) {
+      float cs[8], sn[8], r[8];
+      const int ci = p * 64 + (sub & 7) * 8;
+      *reinterpret_cast<f32x4_t*>(cs) = *reinterpret_cast<const f32x4_t*>(cos_t + ci);
+      *reinterpret_cast<f32x4_t*>(cs + 4) = *reinterpret_cast<const f32x4_t*>(cos_t + ci + 4);
+      *reinterpret_cast<f32x4_t*>(sn) = *reinterpret_cast<const f32x4_t*>(sin_t + ci);
+      *reinterpret_cast<f32x4_t*>(sn + 4) = *reinterpret_cast<const f32x4_t*>(sin_t + ci + 4);
+      head_norm_rope(x, ldg16((gi == kSplitHeads ? k_norm : q_norm) + sub * 8), cs, sn,
+                     eps, sub < 8, r);
+      x = u32x4_t{pack2(r[0], r[1]), pack2(r[2], r[3]), pack2(r[4], r[5]), pack2(r[6], r[7])};
+    }
+    *reinterpret_cast<u32x4_t*>(&l.qs[gi * kSplitQRow + sub * 8]) = x;
+    if (gi >= kSplitHeads && split == 0 && z == 0)
+      *reinterpret_cast<u32x4_t*>((gi == kSplitHeads ? k_cache : v_cache) + cbase +
+                                  (size_t)p * kHd + sub * 8) = x;
   }
+  if (b0 < r1) load_v(s0, b0);
   __syncthreads();
-  u32x4_t qf[4];  // head R, columns 8 (4m + kb)
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-    qf[m] = *reinterpret_cast<const u32x4_t*>(&qs[R * kSplitQRow + 32 * m + 8 * kb]);
   const float sl2 = scale * 1.4426950408889634f;  // scores in log2 units
-  float m = -INFINITY, l = 0.f;                    // head R's running max and sum
+  float m = -INFINITY, lsum = 0.f;                 // head R's running max and sum
   f32x4_t o[8];                                    // o[i][r]: head 4kb + r, column 8R + i
 #pragma unroll
   for (int i = 0; i < 8; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -1180,34 +1211,35 @@ __global__ __launch_bounds__(kSplitWaves * 64, 3) void gqa_split_kernel(
       // the last rows: the new one comes from LDS, and those past it, which
       // hold whatever the cache held, are zeroed
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-        if (b + 16 * u + R == n - 1)
+      for (int q = 0; q < 4; ++q) {
+        const u32x4_t kn = *reinterpret_cast<const u32x4_t*>(
+            &l.qs[kSplitHeads * kSplitQRow + 32 * q + 8 * kb]);
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
-            s.kr[u][q] = *reinterpret_cast<const u32x4_t*>(
-                &qs[kSplitHeads * kSplitQRow + 32 * q + 8 * kb]);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int row = b + vrow(j);
-        if (row == n - 1)
-          s.vr[j] = *reinterpret_cast<const u32x4_t*>(&qs[(kSplitHeads + 1) * kSplitQRow + 8 * R]);
-        else if (row >= n)
-          s.vr[j] = u32x4_t{0u, 0u, 0u, 0u};
+        for (int u = 0; u < 2; ++u)
+          s.kr[u][q] = b + 16 * u + R == n - 1 ? kn : s.kr[u][q];
       }
     }
+    // q from LDS in each step (head R, columns 8 (4q + kb)): 16 registers for
+    // a fourth wave per SIMD
+    int qo = R * kSplitQRow + 8 * kb;
+    asm volatile("" : "+v"(qo));
     float pv[8];
     float mx = -INFINITY;
+    f32x4_t sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      f32x4_t a = {0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < 4; ++q) {
+      const u32x4_t qf = *reinterpret_cast<const u32x4_t*>(&l.qs[qo + 32 * q]);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) a = mfma16x16x32_bf16(s.kr[u][q], qf[q], a);
+      for (int u = 0; u < 2; ++u) sc[u] = mfma16x16x32_bf16(s.kr[u][q], qf, sc[u]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        pv[4 * u + r] = b + 16 * u + 4 * kb + r < n ? a[r] * sl2 : -INFINITY;
+        pv[4 * u + r] = b + 16 * u + 4 * kb + r < n ? sc[u][r] * sl2 : -INFINITY;
         mx = fmaxf(mx, pv[4 * u + r]);
       }
-    }
     const float mn = fmaxf(m, rows4_max(mx));
     const float ref = mn == -INFINITY ? 0.f : mn;
     const float f = __builtin_amdgcn_exp2f(m - ref);
@@ -1229,8 +1261,17 @@ __global__ __launch_bounds__(kSplitWaves * 64, 3) void gqa_split_kernel(
         pv[j] -= __uint_as_float(a & 0xffff0000u);
         pv[j + 1] -= __uint_as_float(e & 0xffff0000u);
       }
-    l = l * f + rows4_sum(ps);
+    lsum = lsum * f + rows4_sum(ps);
     m = mn;
+    if (b + kSplitStep >= n) {
+      const u32x4_t vn =
+          *reinterpret_cast<const u32x4_t*>(&l.qs[(kSplitHeads + 1) * kSplitQRow + 8 * R]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int row = b + vrow(j);
+        s.vr[j] = row < n - 1 ? s.vr[j] : row == n - 1 ? vn : u32x4_t{0u, 0u, 0u, 0u};
+      }
+    }
     float fr[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) fr[r] = __shfl(f, 4 * kb + r);
@@ -1245,102 +1286,119 @@ __global__ __launch_bounds__(kSplitWaves * 64, 3) void gqa_split_kernel(
       for (int r = 0; r < 4; ++r) o[i][r] *= fr[r];
 #pragma unroll
       for (int c = 0; c < 3; ++c) o[i] = mfma16x16x32_bf16(pa[c], vb, o[i]);
+      if (i & 1) __builtin_amdgcn_sched_barrier(0);
     }
   };
   constexpr int kRound = kSplitWaves * kSplitStep;
-  for (int b = b0; b < r1; b += kRound) {
+  for (int b = b0; b < r1;) {
     step(s0, b);
-    if (b + kRound < r1) load(s0, b + kRound);
+    b += kRound;
+    if (b >= r1) break;
+    load_k(s0, b);
+    load_v(s0, b);
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    float* dst = &om[w][4 * kb + r][8 * R];
+    float* dst = &l.om[w][4 * kb + r][8 * R];
     *reinterpret_cast<f32x4_t*>(dst) = f32x4_t{o[0][r], o[1][r], o[2][r], o[3][r]};
     *reinterpret_cast<f32x4_t*>(dst + 4) = f32x4_t{o[4][r], o[5][r], o[6][r], o[7][r]};
   }
   if (kb == 0) {
-    ms[w][R] = m;
-    ls[w][R] = l;
+    l.ms[w][R] = m;
+    l.ls[w][R] = lsum;
   }
   __syncthreads();
-  // the waves' states of head gi, columns 8 sub .. +8
-  if (gi < heads) {
-    float M = -INFINITY;
+  // The waves' states of head h, columns 4 c4 .. +4 (32 lanes per head).
+  const int h = tid >> 5, c4 = tid & 31;
+  const int used = (n + chunk - 1) / chunk;
+  float M = -INFINITY, den = 0.f;
+  f32x4_t a = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int q = 0; q < kSplitWaves; ++q) M = fmaxf(M, ms[q][gi]);
-    const float ref = M == -INFINITY ? 0.f : M;
-    float den = 0.f;
-    f32x4_t a = {0.f, 0.f, 0.f, 0.f}, e = a;
+  for (int q = 0; q < kSplitWaves; ++q) M = fmaxf(M, l.ms[q][h]);
+  const float ref = M == -INFINITY ? 0.f : M;
 #pragma unroll
-    for (int q = 0; q < kSplitWaves; ++q) {
-      const float f = __builtin_amdgcn_exp2f(ms[q][gi] - ref);  // waves without rows: 2^-inf = 0
-      den += f * ls[q][gi];
-      a += f * *reinterpret_cast<const f32x4_t*>(&om[q][gi][8 * sub]);
-      e += f * *reinterpret_cast<const f32x4_t*>(&om[q][gi][8 * sub + 4]);
+  for (int q = 0; q < kSplitWaves; ++q) {
+    const float f = __builtin_amdgcn_exp2f(l.ms[q][h] - ref);  // waves without rows: 2^-inf = 0
+    den += f * l.ls[q][h];
+    a += f * *reinterpret_cast<const f32x4_t*>(&l.om[q][h][4 * c4]);
+  }
+  if (used > 1) {
+    // The last of the token's workgroups adds the splits up.  What the others
+    // wrote goes past the L2s, which are one per XCD.
+    float* recs = sa.part + ((size_t)t * nh + h0 + h) * splits * kSplitRec;
+    if (h < heads) {
+      float* rec = recs + (size_t)split * kSplitRec;
+      st8_coh(rec + 4 + 4 * c4, __float_as_uint(a[0]), __float_as_uint(a[1]));
+      st8_coh(rec + 6 + 4 * c4, __float_as_uint(a[2]), __float_as_uint(a[3]));
+      if (c4 == 0) st8_coh(rec, __float_as_uint(M), __float_as_uint(den));
+      __builtin_amdgcn_s_waitcnt(0);
     }
-    float* rec = part + (((size_t)t * nh + h0 + gi) * splits + split) * kSplitRec;
-    *reinterpret_cast<f32x4_t*>(rec + 4 + 8 * sub) = a;
-    *reinterpret_cast<f32x4_t*>(rec + 8 + 8 * sub) = e;
-    if (sub == 0) {
-      rec[0] = M;
-      rec[1] = den;
+    __syncthreads();
+    if (tid == 0) {
+      int* mine = sa.tickets + (size_t)(t * sa.zh + z) * kvh + g;
+      l.ticket = __hip_atomic_fetch_add(mine, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (l.ticket == used - 1)
+        __hip_atomic_store(mine, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    __syncthreads();
+    if (l.ticket != used - 1) return;
+    // every split's max and sum in lane s of the 32, and 8 splits' columns in
+    // flight at a time (splits past the rows load the last one and weigh 0)
+    const int hh = min(h, heads - 1);
+    const float* rs = sa.part + ((size_t)t * nh + h0 + hh) * splits * kSplitRec;
+    const uint64_t ml = __hip_atomic_load(
+        reinterpret_cast<const uint64_t*>(rs + (size_t)min(c4, used - 1) * kSplitRec),
+        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    constexpr int U = 8;
+    u32x4_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      v[u] = ld16_coh(rs + (size_t)min(u, used - 1) * kSplitRec + 4 + 4 * c4);
+    const float ms = c4 < used ? __uint_as_float((uint32_t)ml) : -INFINITY;
+    M = ms;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) M = fmaxf(M, __shfl_xor(M, off));
+    const float f = __builtin_amdgcn_exp2f(ms - (M == -INFINITY ? 0.f : M));
+    den = c4 < used ? f * __uint_as_float((uint32_t)(ml >> 32)) : 0.f;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) den += __shfl_xor(den, off);
+    a = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int q0 = 0; q0 < used; q0 += U) {
+      if (q0 > 0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          v[u] = ld16_coh(rs + (size_t)min(q0 + u, used - 1) * kSplitRec + 4 + 4 * c4);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float fs = __shfl(f, (lane & 32) + min(q0 + u, used - 1));
+        if (q0 + u < used) a += fs * __builtin_bit_cast(f32x4_t, v[u]);
+      }
+    }
+  }
+  if (h < heads) {
+    const float inv = 1.0f / den;
+    uint32_t* dst = reinterpret_cast<uint32_t*>(out + ((size_t)t * nh + h0 + h) * kHd + 4 * c4);
+    dst[0] = pack2(a[0] * inv, a[1] * inv);  // 4-byte aligned
+    dst[1] = pack2(a[2] * inv, a[3] * inv);
   }
 }
 
-// grid (c, nh), 256 threads: 32-lane group i adds up splits i, i + 8, ... of
-// its head (four columns per lane), the groups meet in LDS.
-__global__ __launch_bounds__(kT) void gqa_merge_kernel(const float* __restrict__ part,
-                                                       const int64_t* __restrict__ pos, int nh,
-                                                       int splits, int L,
-                                                       uint16_t* __restrict__ out) {
-  __shared__ __align__(16) float acc[8][kHd];
-  __shared__ float den[8];
-  const int t = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, i = tid >> 5, c = 4 * (tid & 31);
-  const float* rec = part + ((size_t)t * nh + h) * splits * kSplitRec;
+// grid (c * zh, kvh, max(splits, heads of a group)).
+__global__ __launch_bounds__(kSplitWaves * 64, 4) void gqa_long_kernel(GQA_PARAMS, SplitArgs sa) {
+  static_assert(kSplitWaves == kGqaWaves, "both forms in one launch");
+  __shared__ union {
+    SplitLds split;
+    GqaLds<kGqaWaves> head;
+  } l;
+  const int t = blockIdx.x / sa.zh, z = blockIdx.x - t * sa.zh, g = blockIdx.y, b = blockIdx.z;
+  const int grp = nh / kvh;
   const long long p = pos[t];
   if (p < 0 || p >= L) return;
-  const int n = (int)p + 1, chunk = split_chunk(n, splits), used = (n + chunk - 1) / chunk;
-  // the first pass's loads all go out together (a split past the rows loads
-  // the first one and is not added)
-  constexpr int U = kSplitMax / 8;
-  f32x4_t v[U];
-  float m[U], l[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const float* r = rec + (size_t)(i + 8 * u < used ? i + 8 * u : 0) * kSplitRec;
-    m[u] = i + 8 * u < used ? r[0] : -INFINITY;
-    l[u] = r[1];
-    v[u] = *reinterpret_cast<const f32x4_t*>(r + 4 + c);
-  }
-  float M = -INFINITY;
-  for (int s = 0; s < used; ++s) M = fmaxf(M, rec[(size_t)s * kSplitRec]);
-  const float ref = M == -INFINITY ? 0.f : M;
-  f32x4_t a = {0.f, 0.f, 0.f, 0.f};
-  float d = 0.f;
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    if (i + 8 * u < used) {
-      const float f = __builtin_amdgcn_exp2f(m[u] - ref);
-      a += f * v[u];
-      d += f * l[u];
-    }
-  }
-  *reinterpret_cast<f32x4_t*>(&acc[i][c]) = a;
-  if (c == 0) den[i] = d;
-  __syncthreads();
-  if (tid < kHd / 2) {
-    float s = 0.f, a0 = 0.f, a1 = 0.f;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      s += den[q];
-      a0 += acc[q][2 * tid];
-      a1 += acc[q][2 * tid + 1];
-    }
-    const float inv = 1.0f / s;
-    *reinterpret_cast<uint32_t*>(out + ((size_t)t * nh + h) * kHd + 2 * tid) =
-        pack2(a0 * inv, a1 * inv);
-  }
+  if (p >= kSplitShort)
+    gqa_part(GQA_ARGS, sa, l.split, t, z, g, b, (int)p + 1);
+  else if (b < min(kSplitHeads, grp - z * kSplitHeads))
+    gqa_head<kGqaWaves, kGqaRows, true>(GQA_ARGS, t, g * grp + z * kSplitHeads + b, l.head);
 }
 
 // ---------------------------------------------------------------------------
@@ -1798,65 +1856,60 @@ extern "C" int sluice_dec_mla_decode(const void* q, int q_stride, const void* kv
 
 namespace {
 
-// Scratch of the split kernels: kSplitRegions regions per GPU, held until the
-// process ends.  A call takes a region for its two launches; the region's
-// event marks their end and the next call's stream waits for it, so calls on
-// any streams and threads are kept apart (a wait on the call's own stream
-// costs nothing on the device).  A call prefers the region its stream used
-// last, then one not used yet, then takes them in turn.  (No event is queried:
-// a query is not allowed while another thread captures a graph.)
-struct SplitRegion {
-  hipEvent_t done = nullptr;
-  hipStream_t last = nullptr;
-  bool used = false;
-};
+// Scratch of the split attention: kSplitRegions regions per GPU, held until the
+// process ends.  The first streams that call take a region each, and the order
+// of a stream's own work keeps its calls apart (hipStreamDestroy waits for the
+// stream's work, so a handle that comes back finds the region idle).  All
+// further streams, and hipStreamPerThread, whose one handle names a stream per
+// thread, share the last region: there each call's stream waits for the event
+// that marks the end of the call before.  (An event costs 3 us of the stream
+// per call; a query instead is not allowed while another thread captures.)
 constexpr int kSplitDevices = 64;
+struct SplitScratch {
+  char* base = nullptr;
+  int* tickets = nullptr;
+  hipStream_t owner[kSplitRegions - 1] = {};
+  int owners = 0;
+  hipEvent_t done = nullptr;  // of the shared region
+  bool shared_used = false;
+};
 std::mutex g_split_mu;
-SplitRegion g_split_region[kSplitDevices][kSplitRegions];
-void* g_split_base[kSplitDevices] = {};
-int g_split_next[kSplitDevices] = {};
+SplitScratch g_split[kSplitDevices];
 
-// Under g_split_mu: a region of the current device the stream may write next,
-// or nullptr.
-float* split_take(int dev, hipStream_t st, SplitRegion** out) {
-  if (g_split_base[dev] == nullptr) {
-    void* p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(split_scratch)) != hipSuccess) return nullptr;
-    for (SplitRegion& r : g_split_region[dev])
-      if (r.done == nullptr &&
-          hipEventCreateWithFlags(&r.done, hipEventDisableTiming) != hipSuccess)
-        return nullptr;
-    g_split_base[dev] = p;
+// Under g_split_mu: the region of the current device that the stream may write
+// next, or -1.
+int split_take(SplitScratch& s, hipStream_t st) {
+  if (s.base == nullptr) {
+    void *p = nullptr, *q = nullptr;
+    if (hipGetSymbolAddress(&p, HIP_SYMBOL(split_scratch)) != hipSuccess ||
+        hipGetSymbolAddress(&q, HIP_SYMBOL(split_tickets)) != hipSuccess ||
+        hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess)
+      return -1;
+    s.tickets = (int*)q;
+    s.base = (char*)p;
   }
-  int pick = -1;
-  for (int i = 0; i < kSplitRegions && pick < 0; ++i) {
-    const SplitRegion& r = g_split_region[dev][i];
-    if (r.used && r.last == st) pick = i;
+  if (st != hipStreamPerThread) {
+    for (int i = 0; i < s.owners; ++i)
+      if (s.owner[i] == st) return i;
+    if (s.owners < kSplitRegions - 1) {
+      s.owner[s.owners] = st;
+      return s.owners++;
+    }
   }
-  for (int i = 0; i < kSplitRegions && pick < 0; ++i)
-    if (!g_split_region[dev][i].used) pick = i;
-  if (pick < 0) {
-    pick = g_split_next[dev];
-    g_split_next[dev] = (pick + 1) % kSplitRegions;
-  }
-  SplitRegion& r = g_split_region[dev][pick];
-  if (r.used && hipStreamWaitEvent(st, r.done, 0) != hipSuccess) return nullptr;
-  *out = &r;
-  return (float*)((char*)g_split_base[dev] + (size_t)pick * kSplitRegionBytes);
+  if (s.shared_used && hipStreamWaitEvent(st, s.done, 0) != hipSuccess) return -1;
+  return kSplitRegions - 1;
 }
 
-// The split kernels where they pay: caches of more than 768 rows, several
-// query heads per kv head.  Not while the stream is captured (a replay would
-// use the region without taking it) and not without a region: -1, the caller
-// launches the one-launch kernel, which takes every shape.
-constexpr int kSplitMinRows = 768;
-
+// The split where it pays: caches of more than 768 rows, several query heads
+// per kv head.  Not while the stream is captured (a replay would use the region
+// without taking it) and not without a region: -1, the caller launches the
+// one-launch kernel, which takes every shape.
 int gqa_split(const void* qkv, const float* qkv_parts, int n_parts, const void* q_norm,
               const void* k_norm, const float* cos_t, const float* sin_t, const int64_t* pos, int c,
               int nh, int kvh, int L, float eps, float scale, void* k_cache, void* v_cache,
               void* out, hipStream_t st) {
   const int grp = nh / kvh, zh = (grp + kSplitHeads - 1) / kSplitHeads;
-  if (L <= kSplitMinRows || grp < 2 || kvh > 65535 || nh > 65535) return -1;
+  if (L <= kSplitShort || grp < 2 || kvh > 65535) return -1;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   int dev = 0;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
@@ -1864,27 +1917,36 @@ int gqa_split(const void* qkv, const float* qkv_parts, int n_parts, const void* 
     return -1;
   }
   if (cap != hipStreamCaptureStatusNone || dev < 0 || dev >= kSplitDevices) return -1;
-  // three workgroups per CU, at least 128 rows each
+  // Two workgroups per CU, at least 256 rows each.  A call of more units than
+  // that is not split: its workgroups use no scratch.
   const long units = (long)c * kvh * zh;
-  const int splits = (int)std::max(1L, std::min({768 / units, (long)kSplitMax, (long)L / 128}));
-  if ((size_t)c * nh * splits * kSplitRec * sizeof(float) > kSplitRegionBytes) return -1;
+  const int splits =
+      (int)std::max(1L, std::min({kSplitUnits / units, (long)kSplitMax, (long)L / 256}));
+  static_assert(kSplitRegionBytes >= (size_t)kSplitUnits * kSplitHeads * kSplitRec * sizeof(float) &&
+                    kSplitTickets >= kSplitUnits,
+                "scratch of the largest split call");
   std::lock_guard<std::mutex> lock(g_split_mu);
-  SplitRegion* region = nullptr;
-  float* part = split_take(dev, st, &region);
-  if (part == nullptr) {
+  SplitScratch& s = g_split[dev];
+  const int region = split_take(s, st);
+  if (region < 0) {
     (void)hipGetLastError();
     return -1;
   }
-  hipLaunchKernelGGL(gqa_split_kernel, dim3(c * zh, kvh, splits), dim3(kSplitWaves * 64), 0, st,
-                     (const uint16_t*)qkv, qkv_parts, n_parts, (const uint16_t*)q_norm,
-                     (const uint16_t*)k_norm, cos_t, sin_t, pos, nh, kvh, zh, L, eps, scale,
-                     (uint16_t*)k_cache, (uint16_t*)v_cache, part);
-  hipLaunchKernelGGL(gqa_merge_kernel, dim3(c, nh), dim3(kT), 0, st, (const float*)part, pos, nh,
-                     splits, L, (uint16_t*)out);
-  const hipError_t launched = hipGetLastError(), marked = hipEventRecord(region->done, st);
-  region->used = true;
-  region->last = st;
-  return (int)(launched != hipSuccess ? launched : marked);
+  const SplitArgs sa{zh, splits, (float*)(s.base + region * kSplitRegionBytes),
+                     s.tickets + region * kSplitTickets};
+  hipLaunchKernelGGL(gqa_long_kernel,
+                     dim3(c * zh, kvh, std::max(splits, std::min(grp, kSplitHeads))),
+                     dim3(kSplitWaves * 64), 0, st, (const uint16_t*)qkv, qkv_parts, n_parts,
+                     (const uint16_t*)q_norm, (const uint16_t*)k_norm, cos_t, sin_t, pos, c, nh,
+                     kvh, L, eps, scale, (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)out,
+                     sa);
+  hipError_t rc = hipGetLastError();
+  if (region == kSplitRegions - 1) {
+    const hipError_t marked = hipEventRecord(s.done, st);
+    s.shared_used = true;
+    if (rc == hipSuccess) rc = marked;
+  }
+  return (int)rc;
 }
 
 }  // namespace
@@ -1911,8 +1973,8 @@ extern "C" int sluice_dec_gqa_decode(const void* qkv, const float* qkv_parts, in
   if (split >= 0) return split;
   hipLaunchKernelGGL((gqa_decode_kernel<kGqaWaves, kGqaRows>), dim3(c, nh),
                      dim3(kGqaWaves * 64), 0, (hipStream_t)stream, (const uint16_t*)qkv,
-                     qkv_parts, n_parts, (const uint16_t*)q_norm, (const uint16_t*)k_norm, cos_t, sin_t, pos, nh, kvh,
-                     L, eps, scale, (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)out);
+                     qkv_parts, n_parts, (const uint16_t*)q_norm, (const uint16_t*)k_norm, cos_t, sin_t, pos, c,
+                     nh, kvh, L, eps, scale, (uint16_t*)k_cache, (uint16_t*)v_cache, (uint16_t*)out);
   return (int)hipGetLastError();
 }
 

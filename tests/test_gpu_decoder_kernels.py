@@ -433,11 +433,11 @@ def test_gqa_decode(L, positions):
 @pytest.mark.parametrize("nh,kvh,L,parts", [(32, 4, 800, 0), (8, 4, 4096, 0), (16, 1, 1056, 3),
                                             (40, 2, 769, 0), (32, 16, 2080, 0)])
 def test_gqa_decode_split_matches_the_one_launch_kernel(nh, kvh, L, parts):
-    """Long caches run split over the rows in two launches; while a stream is
-    captured the one-launch kernel runs.  Both keep the softmax in fp32, so the
-    bf16 outputs are at most one rounding apart (2^-8); the cache rows have the
-    same bits.  Rows past a position hold NaN: they have no weight.  Positions
-    outside the cache write nothing."""
+    """Long contexts run split over the rows; while a stream is captured the
+    one-launch kernel runs.  Both keep the softmax in fp32, so the bf16 outputs
+    are at most one rounding apart (2^-8), and the same for contexts that are
+    not split; the cache rows have the same bits.  Rows past a position hold
+    NaN: they have no weight.  Positions outside the cache write nothing."""
     lib, check = _lib()
     hd = 128
     positions = [0, 1, 31, 32, 127, 128, 129, 511, L - 1, -1, L]
@@ -485,8 +485,58 @@ def test_gqa_decode_split_matches_the_one_launch_kernel(nh, kvh, L, parts):
             assert (outs[0][t] == 7.0).all() and (ref[t] == 7.0).all()
             continue
         assert _rel(outs[0][t], ref[t].float().cpu()) <= 2.0 ** -8, (t, p)
+        assert p >= 768 or torch.equal(outs[0][t], ref[t]), (t, p)
         assert torch.equal(k1[t, :, p], k2[t, :, p]) and torch.equal(v1[t, :, p], v2[t, :, p])
         assert torch.isnan(k1[t, :, p + 1:]).all() and torch.equal(k1[t, :, :p], k[t, :, :p])
+
+
+@pytest.mark.parametrize("c,nh,kvh,L", [
+    (1, 32, 4, 4096),    # 16 splits: 2048 rows and more in two rounds of merging loads
+    (3, 4, 2, 1300),     # 5 splits
+    (60, 32, 4, 1100),   # 2 splits
+    (130, 32, 4, 800),   # more units than workgroups are wanted: not split
+    (2, 40, 1, 2000),    # three groups of query heads, the last of 8
+])
+def test_gqa_decode_at_the_line_and_over_the_splits(c, nh, kvh, L):
+    """Contexts around the 768-row line, the splits' edges and the whole cache,
+    against attention in fp64; every call finds the tickets as the one before
+    left them, so each is made three times."""
+    lib, check = _lib()
+    hd = 128
+    g = torch.Generator(device=DEV).manual_seed(c + L)
+
+    def rand(shape):
+        return torch.randn(shape, generator=g, device=DEV).bfloat16()
+
+    edges = [766, 767, 768, 769, 1023, 1024, 1279, 1280, 2047, 2048, L - 1]
+    pos = [min(edges[(t + c) % len(edges)], L - 1) for t in range(c)]
+    if c == 1:
+        pos = [L - 1]
+    qkv, k, v = rand((c, (nh + 2 * kvh) * hd)), rand((c, kvh, L, hd)), rand((c, kvh, L, hd))
+    w = torch.ones(hd, dtype=torch.bfloat16, device=DEV)
+    cos_t, sin_t = (a.to(DEV) for a in _tables(L, hd, 1e6))
+    pos_d = torch.tensor(pos, device=DEV)
+    outs = []
+    for _ in range(3):
+        out = torch.empty((c, nh * hd), dtype=torch.bfloat16, device=DEV)
+        check(lib.sluice_dec_gqa_decode(
+            qkv.data_ptr(), None, 0, w.data_ptr(), w.data_ptr(), cos_t.data_ptr(),
+            sin_t.data_ptr(), pos_d.data_ptr(), c, nh, kvh, hd, L, 1e-6, hd ** -0.5, k.data_ptr(),
+            v.data_ptr(), out.data_ptr(), _st()), "gqa_decode")
+        outs.append(out)
+    torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    q = qkv[:, :nh * hd].double().view(c, nh, hd)
+    q = q * torch.rsqrt(q.square().mean(-1, keepdim=True) + 1e-6)
+    for t in sorted(set(range(0, c, 7)) | {c - 1}):
+        p = pos[t]
+        a, b = q[t].chunk(2, dim=-1)
+        cs, sn = cos_t[p].double(), sin_t[p].double()
+        qr = torch.cat([a * cs - b * sn, b * cs + a * sn], dim=-1).bfloat16().double()
+        for h in range(nh):
+            kc, vc = (x[t, h // (nh // kvh), :p + 1].double() for x in (k, v))
+            want = torch.softmax((kc @ qr[h]) * hd ** -0.5, dim=0) @ vc
+            assert _rel(outs[0][t, h * hd:(h + 1) * hd], want.float().cpu()) <= TOL, (t, h)
 
 
 def test_gqa_decode_split_keeps_infinities():
