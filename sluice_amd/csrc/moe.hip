@@ -675,17 +675,15 @@ __global__ __launch_bounds__(kThreads) void moe_gemm1_kernel(const uint16_t* __r
   }
 }
 
-// gemm1 of a small call that has no plan yet (P <= kSelfPairs pairs, no slot
-// of the map may stream): every workgroup groups the pairs by itself -- one pair
-// per thread, every 16th pair of a slot leads a block -- and one more workgroup, the last, writes the plan that gemm2 and
-// the combine read.  The align launch goes (4.9 us and a launch gap) for two
-// dependent loads (ids, map) and five barriers at the head of each workgroup.
-// Replayed calls, with the align launch and without: V2-Lite 39.3 / 36.6 us
-// for one token, 78.9 / 77.8 for 8, 91.5 / 92.6 for 12; Qwen3 30.0 / 26.9 for
-// one, 66.1 / 64.1 for 12 (96 pairs, the line), 73.2 / 72.9 for 16; V3 fp8 217
-// / 214 for 8.  (Counting each pair's rank against all the others' slots
-// instead of by LDS atomics: 77 us for 12 tokens.)  The shared blocks come
-// first, since their number is known.
+// gemm1 of a small call that has no plan yet (see self_plan; no slot of the map
+// may stream): every workgroup groups the pairs by itself -- one pair per
+// thread, every 16th pair of a slot leads a block -- and one more workgroup,
+// the last, writes the plan that gemm2 and the combine read.  The align launch
+// goes (4.9 us and a launch gap) for two dependent loads (ids, map) and five
+// barriers at the head of each workgroup.  (Counting each pair's rank against
+// all the others' slots instead of by LDS atomics: 77 against 64 us for 12
+// tokens of the Qwen3 shape.)  The shared blocks come first, since their number
+// is known.
 constexpr int kSelfPairs = 96;
 static_assert(kSelfPairs <= kThreads, "a pair per thread");
 
@@ -1189,6 +1187,23 @@ int launch_tiles(const TileArgs& a, long tiles, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// Whether a call without a plan groups its pairs in gemm1.  Every workgroup of
+// the launch does, also those that the largest plan of the call would need and
+// this one does not, so the calls that gain have few workgroups, of long items
+// (fp8), and no slot with more than one block (up to 16 tokens; a slot's
+// further blocks are told one by one).  Even / Zipf routing, with the align
+// launch and without: V2-Lite over 48 slots 31.0 / 28.3 and 31.1 / 28.3 us for
+// one token, 127.5 / 123.3 and 86.7 / 86.6 for 10 (7040 workgroups), 119.0 /
+// 118.3 and 74.9 / 76.2 for 12 (8448); OLMoE 105.9 / 101.8 and 66.8 / 66.1 for
+// 12 (6144); Qwen3 114 / 108 and 58.0 / 55.9 for 12 (96 pairs), and the same
+// for 16; DeepSeek-V3 fp8 428 / 421 and 212 / 207 for 12 (13824).
+template <bool FP8>
+bool self_plan(const CallShape& cs, int n_sh) {
+  const int P = cs.T * cs.k;
+  return P <= kSelfPairs && cs.T <= kBM &&
+         (long)(P + n_sh * cs.T) * (cs.I / 16) <= (FP8 ? 2 : 1) * 7168;
+}
+
 template <bool FP8, int BM>
 int run_tiles(const TileArgs& a, long tiles, hipStream_t st) {
   const int rc = launch_tiles<typename TileFor<FP8, true, BM>::type>(a, tiles, st);
@@ -1244,7 +1259,8 @@ int run_experts(const void* x, const ExpertW& W, const float* tw, const int32_t*
   const int bm = plan == nullptr ? tile_pairs<FP8>(cs, E, S, Ww.I_s) : 0;
   if (bm > 0)
     return run_tiled<FP8>(x, Ww, tw, ti, map, cs, E, S, n_sh, bm, scale, shared, w, out, st);
-  const bool self = plan == nullptr && Ww.wait.pending == nullptr && P <= kSelfPairs;
+  const bool self =
+      plan == nullptr && Ww.wait.pending == nullptr && self_plan<FP8>(cs, n_sh);
   if (self) {
     plan = w.plan;
   } else if (plan == nullptr) {

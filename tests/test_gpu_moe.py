@@ -643,11 +643,14 @@ def test_function_modes_and_lazy_views_go_through_the_op():
     (1, 1, 1, 1, "even"),          # one pair
     (1, 6, 64, 48, "even"),
     (12, 8, 128, 96, "even"),      # 96 pairs: the largest call that plans itself
-    (97, 1, 64, 64, "even"),       # 97 pairs: the align launch
+    (97, 1, 64, 64, "even"),       # the align launch
     (31, 3, 4, 4, "even"),         # about 23 pairs per slot: a block and a rest
     (48, 2, 16, 16, "one"),        # every pair to one expert: six full blocks
     (9, 8, 512, 512, "even"),
     (9, 4, 16, 8, "outside"),      # no pair is resident
+    (12, 8, 16, 16, "one"),        # 96 pairs of 12 tokens to one expert: six blocks
+    (16, 6, 16, 16, "even"),
+    (17, 5, 16, 16, "even"),       # more tokens than a block: the align launch
 ])
 @pytest.mark.parametrize("fp8", [False, True])
 def test_small_calls_plan_themselves(T, k, E, S, how, fp8):
