@@ -1126,15 +1126,21 @@ struct TileFor<false, G1, 128> {
   using type = TileCfg<false, G1, 256, 128, 8, 1, 3>;
 };
 
-// Pairs per tile, or 0 for the decode kernels, from the mean pairs per slot.
-// The decode kernels read an expert's weights once per 16 of its tokens and
-// so win while most experts have one block.  Whole calls in us, decode
-// kernels / tiles, even and Zipf routing: V2-Lite over 48 slots 161 / 176 and
-// 176 / 180 at 8 pairs per slot, 177 / 175 and 207 / 174 at 12; Qwen3 222 /
-// 225 and 187 / 161 at 8, 256 / 229 and 243 / 178 at 12; V3 fp8 422 / 449 at
-// 4, 610 / 559 at 8.  Larger tiles reuse the weights more and pad more: 64 /
-// 128 pairs gave 246 / 249 at 32 per slot and 300 / 279 at 64 (Qwen3), 287 /
-// 244 at 128 (V2-Lite); fp8 32 / 64 pairs 592 / 637 at 16, 672 / 657 at 24.
+// Pairs per tile, or 0 for the decode kernels.  Those read an expert's weights
+// once per 16 of its tokens and so win while most experts have one block: the
+// line is a number of pairs per expert (where only some experts are resident,
+// evenly routed pairs fall on the others too), set where even routing, the worst
+// case, gains on every shape.  Whole calls, decode kernels / tiles in us, even
+// and Zipf routing, at pairs per expert: V2-Lite over 48 slots 175 / 191 and 200
+// / 184 at 9, 192 / 194 and 242 / 194 at 12, 216 / 194 and 221 / 192 at 14; Qwen3
+// over 96 slots 179 / 191 and 210 / 187 at 10, 218 / 194 and 257 / 191 at 14;
+// OLMoE over 64 slots 160 / 169 and 169 / 155 at 12, 181 / 170 and 189 / 175 at
+// 14; Qwen1.5-MoE over 60 slots 205 / 212 and 208 / 178 at 12.8, 231 / 213 and
+// 229 / 172 at 14.9; DeepSeek-V3 fp8 over 64 of 256 slots 495 / 552 and 679 / 556
+// at 3, 557 / 569 and 891 / 612 at 5, 605 / 581 and 955 / 612 at 6.
+// Larger tiles reuse the weights more and pad more, by pairs per slot: 64 / 128
+// pairs gave 246 / 249 at 32 per slot and 300 / 279 at 64 (Qwen3), 287 / 244 at
+// 128 (V2-Lite); fp8 32 / 64 pairs 592 / 637 at 16, 672 / 657 at 24.
 //
 // A call over few slots must also fill the device: the tiles are taken where
 // they make at least one item per CU.  And a lane's offsets into the tokens
@@ -1144,7 +1150,7 @@ int tile_pairs(const CallShape& cs, int E, int S, int shared_I) {
   const int slots = std::min(E, S), P = cs.T * cs.k;
   const size_t rows = std::max<size_t>(cs.T, std::max<size_t>(2 * cs.I, 2 * (size_t)shared_I));
   if (rows * cs.H * 2 > UINT32_MAX) return 0;
-  if (P <= SLUICE_MAX_PAIRS && P < (FP8 ? 6 : 10) * slots) return 0;
+  if (P < (FP8 ? 6 : 14) * E) return 0;
   const int bm = FP8 ? (P < 20 * slots ? 32 : 64) : P < 64 * slots ? 64 : 128;
   const int ch = bm == 128 ? 256 : 128;
   const long items = (long)std::max(P / bm, slots) * std::min(2 * cs.I / ch, cs.H / ch);
@@ -1214,7 +1220,7 @@ int run_tiles(const TileArgs& a, long tiles, hipStream_t st) {
 // The tiled product: sort, gemm1, gemm2, combine.  The sorted call sits in
 // the workspace's plan area, which is always larger (checked): with up to 4
 // shared groups the records, order and flags take at most 5 ints per pair
-// and 24 more, the plan 19 per pair and 4, and a tiled call has 12 pairs.
+// and 24 more, the plan 19 per pair and 4.
 template <bool FP8>
 int run_tiled(const void* x, const ExpertW& W, const float* tw, const int32_t* ti,
               const int32_t* map, const CallShape& cs, int E, int S, int n_sh, int bm, float scale,

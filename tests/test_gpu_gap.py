@@ -860,7 +860,7 @@ def test_tiled_product_waits_for_rows_in_flight(monkeypatch, kind):
     bytes, which arrive with the weights (the gap kernel copies none)."""
     from sluice_amd import _lib, ops
 
-    E, S, k, H, I, T = 96, 32, 4, 1152, 640, 96
+    E, S, k, H, I, T = 96, 32, 4, 1152, 640, 352  # 14 pairs per expert and more
     print(f"tiles over rows in flight: {kind}", flush=True)
     monkeypatch.setenv("SLUICE_STAGE_ROWS", "0")
     monkeypatch.setenv("SLUICE_CODEC", "1" if kind == "bf16-coded" else "0")

@@ -417,11 +417,13 @@ def _in_slices(args, kw, n):
 
 
 @pytest.mark.parametrize("T,H,I,Is,E,S,k,frac,fp8", [
-    (80, 1088, 448, 448, 40, 40, 5, 0.8, False),    # 10 pairs per slot: the smallest, odd sizes
+    (112, 1088, 448, 448, 40, 40, 5, 0.8, False),   # 14 pairs per expert: the smallest, odd sizes
+    (111, 1088, 448, 448, 40, 40, 5, 0.8, False),   # below the line
     (257, 1088, 448, 896, 64, 40, 5, 0.8, False),   # 64-pair tiles, partial ones
     (801, 2112, 1472, 0, 40, 40, 5, 1.0, False),    # 128-pair tiles
     (1000, 1088, 448, 448, 40, 40, 5, 0.8, False),  # over 4096 pairs: one prefill call
-    (600, 64, 64, 0, 512, 512, 8, 0.9, False),      # over 4096 pairs, few per slot, one K chunk
+    (900, 64, 64, 0, 512, 512, 8, 0.9, False),      # over 4096 pairs, few per slot, one K chunk
+    (600, 64, 64, 0, 512, 512, 8, 0.9, False),      # below the line in one call
     (301, 2048, 1024, 0, 16, 16, 16, 1.0, False),   # every token to every expert
     (300, 1088, 448, 448, 64, 40, 5, 0.0, False),   # nothing routed is resident
     (72, 1152, 640, 640, 48, 48, 4, 0.8, True),     # fp8, 32-pair tiles: the smallest
@@ -564,9 +566,9 @@ def test_tiled_product_over_a_map_whose_slots_streamed():
     try:
         g = torch.Generator(device=DEV).manual_seed(6)
         layer(torch.randn((4, H), generator=g, device=DEV).to(torch.bfloat16))  # fills slots
-        x = torch.randn((64, H), generator=g, device=DEV).to(torch.bfloat16)
-        ids = torch.randint(0, E, (64, k), generator=g, device=DEV, dtype=torch.int32)
-        tw = torch.rand((64, k), generator=g, device=DEV)
+        x = torch.randn((96, H), generator=g, device=DEV).to(torch.bfloat16)
+        ids = torch.randint(0, E, (96, k), generator=g, device=DEV, dtype=torch.int32)
+        tw = torch.rand((96, k), generator=g, device=DEV)
         args = [x, layer.w13_weight, layer.w2_weight, tw, ids]
         kw = dict(global_num_experts=E, expert_map=layer.expert_map)
         got = ops.fused_experts(*args, **kw)
