@@ -86,9 +86,10 @@ inline long tile_bound(int P, int slots, int T, int n_sh, int bm) {
 // still stream), cut into tiles of at most bm pairs.  The order of the pairs
 // inside a slot is whatever the LDS atomics make it: a pair's product does
 // not depend on its column.  One workgroup, latency-bound: a thread keeps its
-// U pairs' slots and ranks in registers between counting and placing, and the
-// pairs are placed in LDS and written out whole (scattered global stores,
-// one line each, took most of the kernel).  P <= U * kSortThreads.
+// U pairs' slots and ranks in registers between counting and placing (at U = 64
+// 84 bytes per lane go to scratch, at 32 32), and the pairs are placed in LDS and
+// written out whole (scattered global stores, one line each, took most of the
+// kernel).  P <= U * kSortThreads.
 template <int U>
 __global__ __launch_bounds__(kSortThreads) void moe_sort_kernel(
     const int32_t* __restrict__ ids, int P, const int32_t* __restrict__ map, int E, int S,

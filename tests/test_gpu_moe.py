@@ -103,6 +103,8 @@ def _moe_case(T, H, I, E, S, k, seed, resident_frac=0.85, use_map=True, scale=1.
     (8, 2048, 1408, 60, 16, 4),     # Qwen1.5-MoE-A2.7B expert shape (60 experts)
     (33, 256, 192, 16, 16, 4),      # > 16 pairs per slot: several blocks per expert
     (5, 64, 128, 8, 8, 2),          # K shorter than the waves: some waves stream nothing
+    (120, 1088, 448, 40, 40, 5),    # the tiled kernels, 64-pair tiles
+    (900, 1088, 448, 40, 40, 5),    # 128-pair tiles, over 4096 pairs
 ])
 def test_fused_experts_bf16(T, H, I, E, S, k):
     print(f"fused bf16 T={T} H={H} I={I} E={E} S={S} k={k}", flush=True)
@@ -338,6 +340,8 @@ def _fp8_case(T, H, I, E, S, k, seed):
     (8, 7168, 2048, 256, 6, 8),     # DeepSeek-V3 expert shape
     (1, 7168, 2048, 256, 4, 8),
     (12, 512, 256, 16, 8, 4),
+    (80, 1152, 640, 48, 48, 4),     # the tiled kernels, 32-pair tiles
+    (400, 1152, 640, 48, 48, 4),    # 64-pair tiles
 ])
 def test_fused_experts_fp8(T, H, I, E, S, k):
     print(f"fused fp8 T={T} H={H} I={I} E={E} S={S} k={k}", flush=True)
@@ -469,6 +473,40 @@ def test_tiled_product_does_not_depend_on_the_slots(fp8):
     assert torch.equal(got, want)
 
 
+def _kernels(call):
+    """Names of the kernels that call() launches."""
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return " ".join(e.key for e in prof.key_averages())
+
+
+@pytest.mark.parametrize("T,H,I,Is,E,S,k,fp8,route", [
+    (10, 64, 1408, 2816, 64, 48, 6, False, "gemm1_self"),   # 7040 workgroups
+    (11, 64, 1408, 2816, 64, 48, 6, False, "align"),        # 7744
+    (16, 128, 256, 0, 16, 16, 6, True, "gemm1_self"),
+    (17, 128, 256, 0, 16, 16, 5, True, "align"),            # a slot may have two blocks
+    (111, 1088, 448, 448, 40, 40, 5, False, "align"),
+    (112, 1088, 448, 448, 40, 40, 5, False, "tile"),        # 14 pairs per expert
+    (178, 1088, 448, 0, 64, 40, 5, False, "align"),         # ... of all, resident or not
+    (180, 1088, 448, 0, 64, 40, 5, False, "tile"),
+    (71, 1152, 640, 640, 48, 48, 4, True, "align"),
+    (72, 1152, 640, 640, 48, 48, 4, True, "tile"),          # 6, fp8
+    (600, 64, 64, 0, 512, 512, 8, False, "align"),          # over 4096 pairs
+    (900, 64, 64, 0, 512, 512, 8, False, "tile"),
+])
+def test_which_kernels_run(T, H, I, Is, E, S, k, fp8, route):
+    """Both sides of each line: other kernels there were measured slower."""
+    from sluice_amd import ops
+
+    args, kw = _tile_case(T, H, I, Is, E, S, k, 1.0, fp8, seed=T)
+    ops.fused_experts(*args, **kw)
+    names = _kernels(lambda: ops.fused_experts(*args, **kw))
+    ran = [r for r in ("gemm1_self", "align", "tile") if f"moe_{r}_kernel" in names]
+    assert ran == [route], names
+
+
 def test_tiled_product_keeps_tokens_apart():
     """A token of NaN and one of infinities change no other token's bits."""
     from sluice_amd import ops
@@ -555,8 +593,9 @@ def test_graphs_replay_after_a_longer_eager_call(monkeypatch):
 
 
 def test_tiled_product_over_a_map_whose_slots_streamed():
-    """A prefill call over the map of a layer whose last gap filled slots
-    waits for them like the decode kernels do, and gives their product."""
+    """A prefill call over a layer's registered map, whose last gap filled
+    slots (all landed by then: the layer's own product waited), gives the
+    decode kernels' product.  Rows in flight: test_gpu_gap.py."""
     from sluice_amd import ops
     from sluice_amd.decoder import SyntheticMoELayer, build_offloaded
 
