@@ -694,12 +694,13 @@ __global__ __launch_bounds__(kMlaWaves * 64) void mla_partial_kernel(
 // whose address does not depend on the position goes out first: the w_uv
 // rows, every split's (max, sum) and the first kMlaPre splits' partial sums
 // (splits past the position are never used, so whatever they hold is
-// harmless: they are selected away, not multiplied by 0).  Each further pass
-// over the splits is a memory round trip: 16 at a time against 8 took the
-// three launches from 19.2 to 18.2 us for 8 tokens of 120 to 1023 rows, from
-// 28.2 to 27.2 for 1000 to 4095 (and from 12.4 to 12.5 for one token of 128 to
-// 383).
-constexpr int kMlaPre = 16;
+// harmless: they are selected away, not multiplied by 0).  The other splits'
+// go out together as soon as the position is known.  The three launches,
+// replayed, with the others 8 at a time behind one another / 16 first and 16
+// behind / now: 11.7 / 12.1 / 11.7 us for one token of 100 to 255 rows, 14.6 /
+// 15.8 / 15.0 for 12; 12.8 / 12.2 / 12.2 for one of 128 to 383; 16.9 / 16.7 /
+// 16.2 for 8 of 120 to 1023; 27.8 / 26.9 / 26.3 for 8 of 1000 to 4095.
+constexpr int kMlaPre = 8;
 __global__ __launch_bounds__(kT) void mla_merge_kernel(const float* __restrict__ part,
                                                        const uint16_t* __restrict__ w_uv,
                                                        const int64_t* __restrict__ pos, int nh,
@@ -732,6 +733,16 @@ __global__ __launch_bounds__(kT) void mla_merge_kernel(const float* __restrict__
   const int n = (int)p + 1;
   const int chunk = mla_chunk(n);
   const int na = (n + chunk - 1) / chunk;
+  f32x2_t pw[kMlaSplit - kMlaPre];
+#pragma unroll
+  for (int s0 = kMlaPre; s0 < kMlaSplit; s0 += kMlaPre) {
+    if (s0 < na) {
+#pragma unroll
+      for (int u = s0; u < s0 + kMlaPre; ++u)
+        pw[u - kMlaPre] =
+            *reinterpret_cast<const f32x2_t*>(rec + (u < na ? u : 0) * sstride + 4 + 2 * tid);
+    }
+  }
   if (tid < 64) {
     const bool ok = tid < na;
     const float M = wave_max(ok ? ms : -INFINITY);
@@ -749,17 +760,15 @@ __global__ __launch_bounds__(kT) void mla_merge_kernel(const float* __restrict__
         v1 += ws[u] * pv[u][1];
       }
     }
-    for (int s0 = kMlaPre; s0 < na; s0 += kMlaPre) {
 #pragma unroll
-      for (int u = 0; u < kMlaPre; ++u) {
-        const int sp = s0 + u < na ? s0 + u : 0;
-        pv[u] = *reinterpret_cast<const f32x2_t*>(rec + sp * sstride + 4 + 2 * tid);
-      }
+    for (int s0 = kMlaPre; s0 < kMlaSplit; s0 += kMlaPre) {
+      if (s0 < na) {
 #pragma unroll
-      for (int u = 0; u < kMlaPre; ++u) {
-        if (s0 + u < na) {
-          v0 += ws[s0 + u] * pv[u][0];
-          v1 += ws[s0 + u] * pv[u][1];
+        for (int u = s0; u < s0 + kMlaPre; ++u) {
+          if (u < na) {
+            v0 += ws[u] * pw[u - kMlaPre][0];
+            v1 += ws[u] * pw[u - kMlaPre][1];
+          }
         }
       }
     }
