@@ -200,7 +200,8 @@ int sluice_fused_experts_fp8(const void* x, const void* w13,
 
 /* The same product for prefill chunks of more than SLUICE_MAX_PAIRS pairs:
  * T*(k + shared_I/I) <= SLUICE_MAX_PREFILL_PAIRS in one call, so that the
- * chunk reads each expert's weights once.  bf16 experts when w13_scale and
+ * chunk reads each expert's weights once.  Its bits are those of the calls
+ * above over slices of the chunk.  bf16 experts when w13_scale and
  * w2_scale are NULL, e4m3fn with 128x128 block scales when both are given.
  * Workspace: sluice_fused_experts_workspace() bytes, as above. */
 int sluice_fused_experts_prefill(const void* x, const void* w13, const float* w13_scale,

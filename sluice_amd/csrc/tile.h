@@ -19,10 +19,11 @@
 // A pair's sums have the decode kernels' order, so its bits depend neither on
 // the size of its call nor on the slot its expert sits in: the products of a
 // chunk meet in the same MFMAs, and K is summed in the decode kernels' parts
-// (their waves), whose sums are added in part order.  The parts cost a second
-// set of accumulators.  (K in one sum, started at an offset of the slot's own
-// so that workgroups do not meet in the same memory channels, measured 216
-// against 226, 574 against 593 and 696 against 705 us for the calls below.)
+// (their waves), whose sums are added in part order.  The second set of
+// accumulators costs no time; what the order rules out is to start K at an
+// offset of the slot's own, so that workgroups do not meet in the same memory
+// channels (217 against 229, 574 against 594 and 696 against 703 us for the
+// calls below).
 //
 // Bound: HBM while the experts have few tokens (the weights are read once;
 // 4.9 TB/s in gemm1 of the V2-Lite call below, the DMA stream alone reaches
