@@ -13,12 +13,12 @@
 #include "stream.h"
 
 // Scratch of the split attention (see SplitScratch): 512 workgroups' sums of 16
-// heads (528 bytes each) and their tickets, which are zero between launches.
+// heads (528 bytes each) and their tickets, two sets of them taken in turn.
 constexpr int kSplitRegions = 4;
 constexpr size_t kSplitRegionBytes = 512 * 16 * 528;
 constexpr int kSplitTickets = 512;
 static __device__ __align__(256) uint8_t split_scratch[kSplitRegions * kSplitRegionBytes];
-static __device__ int split_tickets[kSplitRegions * kSplitTickets];
+static __device__ int split_tickets[kSplitRegions * 2 * kSplitTickets];
 
 namespace {
 
@@ -1121,12 +1121,15 @@ __host__ __device__ inline int split_chunk(int n, int splits) {
   return ((n + splits - 1) / splits + kRound - 1) / kRound * kRound;
 }
 
-// zh: groups of 16 query heads per kv head; tickets [c * zh * kvh], zero
-// between launches.
+// zh: groups of 16 query heads per kv head; tickets [c * zh * kvh]: zero, and
+// zero again after the launch; next: the set that the region's next launch
+// takes, cleared here, so that a launch whose positions changed while it ran
+// spoils no later one.
 struct SplitArgs {
   int zh, splits;
   float* part;
   int* tickets;
+  int* next;
 };
 
 struct SplitLds {
@@ -1403,6 +1406,8 @@ __global__ __launch_bounds__(kSplitWaves * 64, 4) void gqa_long_kernel(GQA_PARAM
   const int t = blockIdx.x / sa.zh, z = blockIdx.x - t * sa.zh, g = blockIdx.y, b = blockIdx.z;
   const int grp = nh / kvh;
   const long long p = pos[t];
+  static_assert(kSplitTickets == kSplitWaves * 64, "a ticket per thread");
+  if (blockIdx.x == 0 && g == 0 && b == 0) sa.next[threadIdx.x] = 0;
   if (p < 0 || p >= L) return;
   if (p >= kSplitShort)
     gqa_part(GQA_ARGS, sa, l.split, t, z, g, b, (int)p + 1);
@@ -1881,6 +1886,7 @@ struct SplitScratch {
   int owners = 0;
   hipEvent_t done = nullptr;  // of the shared region
   bool shared_used = false;
+  unsigned turn[kSplitRegions] = {};
 };
 std::mutex g_split_mu;
 SplitScratch g_split[kSplitDevices];
@@ -1918,7 +1924,8 @@ int gqa_split(const void* qkv, const float* qkv_parts, int n_parts, const void* 
               int nh, int kvh, int L, float eps, float scale, void* k_cache, void* v_cache,
               void* out, hipStream_t st) {
   const int grp = nh / kvh, zh = (grp + kSplitHeads - 1) / kSplitHeads;
-  if (L <= kSplitShort || grp < 2 || kvh > 65535) return -1;
+  // (a lane's offsets into one kv head's rows are 32-bit)
+  if (L <= kSplitShort || L >= 1 << 24 || grp < 2 || kvh > 65535) return -1;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   int dev = 0;
   if (hipStreamIsCapturing(st, &cap) != hipSuccess || hipGetDevice(&dev) != hipSuccess) {
@@ -1941,8 +1948,10 @@ int gqa_split(const void* qkv, const float* qkv_parts, int n_parts, const void* 
     (void)hipGetLastError();
     return -1;
   }
+  int* const sets = s.tickets + region * 2 * kSplitTickets;
+  const unsigned set = s.turn[region]++ & 1;
   const SplitArgs sa{zh, splits, (float*)(s.base + region * kSplitRegionBytes),
-                     s.tickets + region * kSplitTickets};
+                     sets + set * kSplitTickets, sets + (set ^ 1) * kSplitTickets};
   hipLaunchKernelGGL(gqa_long_kernel,
                      dim3(c * zh, kvh, std::max(splits, std::min(grp, kSplitHeads))),
                      dim3(kSplitWaves * 64), 0, st, (const uint16_t*)qkv, qkv_parts, n_parts,
