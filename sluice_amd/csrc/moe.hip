@@ -1116,7 +1116,7 @@ int launch_combine(const float* partial, const int32_t* valid, const float* topk
 // tile), 128 weight rows per four-wave workgroup and stages that let two
 // workgroups share a CU; beyond, one eight-wave workgroup of 256 rows, which
 // reads the tokens half as often (gemm1 at 4096 tokens of the Qwen3 shape:
-// 306 us against 325 for 128 x 128 tiles, 386 for 128 x 64).
+// 306 us against 325 for 128 x 128 tiles, 386 for 128 x 64, with K in one sum).
 template <bool FP8, bool G1, int BM>
 struct TileFor {
   using type = TileCfg<FP8, G1, 128, BM, 4, 1, FP8 && BM == 64 ? 2 : 3>;

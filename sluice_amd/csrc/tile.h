@@ -26,7 +26,7 @@
 // calls below).
 //
 // Bound: HBM while the experts have few tokens (the weights are read once;
-// 4.9 TB/s in gemm1 of the V2-Lite call below, the DMA stream alone reaches
+// 4.2 TB/s in gemm1 of the V2-Lite call below, the DMA stream alone reaches
 // 6.2), the operand traffic out of L2 beyond (a 4096-token call runs no faster
 // with the LDS reads scheduled between the products).  Whole calls, timed in
 // turn with the decode kernels, same bits: Qwen3 shape, 4096 tokens, 4076 ->
